@@ -96,9 +96,8 @@ struct CtlArgs
     std::uint64_t* stats     = nullptr; ///< kStatSlots copies of kNumStats counters, or null
 };
 
-/// @brief Input partitions of a hybrid run: one per XCD, so that waves
-/// (dispatched round-robin over the 8 XCDs) mostly claim from their own
-/// counter and their own L2.
+/// @brief Ranges of the claimed input of a hybrid run (see Dealt): one per
+/// XCD, over which workgroups are dispatched round-robin.
 inline constexpr std::uint32_t kRanges = 8;
 
 /// @brief Hybrid control block, resident in device memory.
@@ -110,17 +109,20 @@ struct alignas(256) Slot64
     std::uint64_t v;
 };
 
+struct alignas(256) Slot32
+{
+    std::uint32_t v;
+};
+
 struct HybridCtl
 {
-    Slot64        next[kRanges];  ///< next unadmitted thread of each range
-    Slot64        end[kRanges];   ///< end of each range
+    Slot32        next[kRanges];  ///< batches claimed of each range
     std::uint32_t batch_next;     ///< batch claim counter of the pass
     std::uint32_t nbatches;       ///< queue batches of the pass
     std::uint32_t parity;         ///< in-queue side of the pass
     std::uint32_t live;           ///< threads queued for the pass
     std::uint32_t passes;         ///< passes run so far
     std::uint32_t done;           ///< set when no thread remains
-    std::uint32_t exhausted;      ///< bit r: range r has no input left (read before claiming)
     std::uint32_t qcount[2][64];  ///< per side, per label queue fill
     std::uint32_t bprefix[65];    ///< batch prefix over labels of the pass
 };
@@ -1034,80 +1036,161 @@ fill_label(std::uint32_t label, Regs<K>& r, const char* q, std::uint64_t qcap,
 // ---------------------------------------------------------------------------
 // hybrid form: pass kernel
 // ---------------------------------------------------------------------------
-/// @brief A wave's private reservoir of unadmitted thread indices.  Refills
-/// draw from it without atomics; it is topped up from the shared input
-/// ranges in guided chunks (large while much input remains, one batch near
-/// the end), preferring the range of the wave's XCD.  Exhausted ranges are
-/// remembered so that they are not polled again.
-struct Reservoir
+/// @brief How a hybrid run's input is dealt to its waves, in batches of 64
+/// threads.
+///
+/// Every claim of input is an atomic at the memory side of all eight XCDs,
+/// about 18 ns each on one counter: when every wave of a full grid claims
+/// every batch, and at the end finds every range empty, a run of a few
+/// batches per wave spends its time on them (1,048,576 fib threads: 330 us,
+/// where the compact form takes 48).  So the first rounds need no claim:
+/// round j gives wave w the batch j * grid + w, and the whole grid moves along
+/// one front, as claimed batches would.  Below four batches per wave, where a
+/// claimed batch would come as late as a dealt one, that is the whole input
+/// (the same run: 62 us); from there on it is one round, or an eighth of the
+/// input: a SIMD serves its oldest wave first, and of twenty waves per CU the
+/// slowest takes about two fifths of the mean (with half the input dealt, the
+/// path tracer's frame waits for those: 8.1 ms instead of 7.6).
+///
+/// The other batches are dealt round-robin to kRanges ranges, each claimed
+/// from by the waves of one residue (workgroups go round-robin over the
+/// XCDs), so that every range is a sample of the whole input and they run dry
+/// together, but for the XCDs' speeds, which differ by 2%: in runs long
+/// enough to notice, a wave whose range is dry tries two others.
+struct Dealt
 {
-    std::uint64_t base      = 0;
-    std::uint32_t count     = 0;
-    std::uint32_t exhausted = 0; ///< bit r: range r has no input left
-    std::uint32_t chunk     = 0; ///< next claim size (0: not sized yet)
+    std::uint32_t batches = 0; ///< of the whole input
+    std::uint32_t rounds  = 0; ///< batches every wave gets without a claim
+    std::uint32_t ranges  = 1;
+    std::uint32_t tries   = 0; ///< ranges of others that a wave tries at the end
+
+    __host__ __device__ Dealt(std::uint64_t n, std::uint32_t grid) :
+        batches(static_cast<std::uint32_t>((n + 63) / 64)), ranges(grid >= kRanges ? kRanges : 1)
+    {
+        const std::uint32_t per = batches / grid;
+        rounds = per < 4 ? (batches + grid - 1) / grid : (per < 16 ? 1 : per / 8);
+        tries  = per < 16 || ranges == 1 ? 0 : 2;
+    }
+
+    /// batches of range @p r
+    __host__ __device__ std::uint32_t
+    claimed(std::uint32_t r, std::uint32_t grid) const
+    {
+        const std::uint64_t dealt = std::uint64_t(rounds) * grid;
+        const std::uint32_t left  = dealt < batches ? batches - static_cast<std::uint32_t>(dealt) : 0;
+        return left > r ? (left - r + ranges - 1) / ranges : 0;
+    }
 };
 
-/// @brief Guided claim size: about half a fair share of what a range still
-/// holds among the waves that draw from it, one batch at least, 512 at most.
-LOOM_DEVICE std::uint32_t
-guided_chunk(std::uint64_t left)
+/// @brief A wave's private reservoir of unadmitted threads: what is left of
+/// the batch in hand, and the batches after it (each `step` after the last).
+struct Reservoir
 {
-    const std::uint64_t share = gridDim.x / kRanges ? gridDim.x / kRanges : 1;
-    const std::uint64_t c     = left / (2 * share);
-    return static_cast<std::uint32_t>(c < 64 ? 64 : (c > 512 ? 512 : c));
+    std::uint32_t base  = 0; ///< first thread left of the batch in hand
+    std::uint32_t count = 0; ///< threads left of it
+    std::uint32_t next  = 0; ///< the next batch
+    std::uint32_t step  = 0;
+    std::uint32_t units = 0; ///< batches after the one in hand
+    std::uint32_t range = 0; ///< the range claimed from
+    std::uint32_t chunk = 0; ///< batches of the next claim, 0 once the range is empty
+    std::uint32_t tries = 0; ///< ranges left to try
+
+    /// Guided claim size: at most half a fair share of the @p left batches of
+    /// the range among its @p share waves (a shift, so that no claim waits
+    /// for a division), 1 to 8.
+    LOOM_DEVICE void
+    size_claim(std::uint32_t left, std::uint32_t share)
+    {
+        const std::uint32_t c = left >> (33 - __builtin_clz((share > 2 ? share : 2) - 1));
+        chunk                 = left == 0 ? 0 : (c < 1 ? 1 : (c > 8 ? 8 : c));
+    }
+};
+
+/// @brief The reservoir of this wave at the start of a pass.  @p taken: the
+/// batches of its range claimed in earlier passes, whose first one dealt the
+/// rounds too.
+LOOM_DEVICE Reservoir
+deal(const Dealt& d, std::uint32_t wave, std::uint32_t grid, bool first_pass, std::uint32_t taken)
+{
+    Reservoir res;
+    res.range                 = wave % d.ranges;
+    res.tries                 = d.tries;
+    res.next                  = wave;
+    res.step                  = grid;
+    res.units                 = first_pass ? d.rounds : 0;
+    const std::uint32_t total = d.claimed(res.range, grid);
+    res.size_claim(taken < total ? total - taken : 0, grid / d.ranges);
+    return res;
 }
 
-/// @brief Take up to @p want consecutive thread indices (wave-uniform).
-LOOM_DEVICE std::uint32_t
-take_input(HybridCtl* ctl, std::uint32_t home, Reservoir& res, std::uint32_t want,
-           std::uint64_t& base)
+/// @brief Put the next batch in hand (claiming more when the reservoir holds
+/// none); count stays 0 once no input is left.
+LOOM_DEVICE void
+next_batch(HybridCtl* ctl, const Dealt& d, std::uint64_t n, Reservoir& res)
 {
-    if(res.count == 0)
+    while(res.units == 0)
     {
         if(res.chunk == 0)
         {
-            const std::uint64_t nx = ctl->next[home].v, en = ctl->end[home].v;
-            res.chunk              = guided_chunk(uniform64(nx < en ? en - nx : 0));
+            if(res.tries == 0) return;
+            // another range, near the end by now: batch by batch
+            --res.tries;
+            res.range = (res.range + 1 + (blockIdx.x / kRanges) % (kRanges - 1)) % kRanges;
+            res.chunk = 1;
         }
-        std::uint64_t b = 0, e = 0;
-        std::uint32_t got = 0, exh = res.exhausted;
-        if(lane_id() == 0)
-        {
-            // ranges another wave found empty: a plain load instead of one
-            // more serialised atomic per wave and range at the end of input
-            exh |= __hip_atomic_load(&ctl->exhausted, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            for(std::uint32_t i = 0; i < kRanges && !got; ++i)
-            {
-                const std::uint32_t r = (home + i) % kRanges;
-                if((exh >> r) & 1u) continue;
-                e                     = ctl->end[r].v;
-                const std::uint64_t k = atomicAdd(
-                    reinterpret_cast<unsigned long long*>(&ctl->next[r].v),
-                    static_cast<unsigned long long>(res.chunk));
-                if(k < e)
-                {
-                    b   = k;
-                    got = static_cast<std::uint32_t>(e - k < res.chunk ? e - k : res.chunk);
-                }
-                else
-                {
-                    exh |= 1u << r;
-                    __hip_atomic_fetch_or(&ctl->exhausted, 1u << r, __ATOMIC_RELAXED,
-                                          __HIP_MEMORY_SCOPE_AGENT);
-                }
-            }
-        }
-        res.base      = uniform64(b);
-        res.count     = uniform(got);
-        res.exhausted = uniform(exh);
-        // guided chunking on what the range still holds
-        res.chunk = guided_chunk(uniform64(e) - (res.base + res.count));
+        const std::uint32_t total = d.claimed(res.range, gridDim.x);
+        std::uint32_t       k     = 0;
+        if(lane_id() == 0) k = atomicAdd(&ctl->next[res.range].v, res.chunk);
+        k         = uniform(k);
+        res.next  = d.rounds * gridDim.x + res.range + k * d.ranges;
+        res.step  = d.ranges;
+        res.units = k >= total ? 0 : (total - k < res.chunk ? total - k : res.chunk);
+        res.size_claim(k < total ? total - k - res.units : 0, gridDim.x / d.ranges);
     }
-    const std::uint32_t g = res.count < want ? res.count : want;
-    base                  = res.base;
-    res.base += g;
-    res.count -= g;
-    return g;
+    if(res.next < d.batches)
+    {
+        res.base  = res.next * 64u;
+        res.count = n - res.base < 64u ? static_cast<std::uint32_t>(n - res.base) : 64u;
+    }
+    res.next += res.step;
+    --res.units;
+}
+
+/// @brief Up to @p want threads from the reservoir (wave-uniform): the rest of
+/// the batch in hand and, if that is not enough, of the one after it.  The
+/// k-th of them is @p at(k).
+struct Taken
+{
+    std::uint32_t count = 0;
+    std::uint32_t head = 0, base = 0, more = 0; ///< head threads from base on, then from more on
+
+    LOOM_DEVICE std::uint32_t
+    at(std::uint32_t k) const
+    {
+        return k < head ? base + k : more + (k - head);
+    }
+};
+
+LOOM_DEVICE Taken
+take_input(HybridCtl* ctl, const Dealt& d, std::uint64_t n, Reservoir& res, std::uint32_t want)
+{
+    Taken t;
+    if(res.count == 0) next_batch(ctl, d, n, res);
+    t.base  = res.base;
+    t.head  = res.count < want ? res.count : want;
+    t.count = t.head;
+    res.base += t.head;
+    res.count -= t.head;
+    if(t.count < want && t.count != 0)
+    {
+        next_batch(ctl, d, n, res);
+        const std::uint32_t g = res.count < want - t.count ? res.count : want - t.count;
+        t.more                = res.base;
+        t.count += g;
+        res.base += g;
+        res.count -= g;
+    }
+    return t;
 }
 
 /// @brief One hybrid pass.  Launched with one wave per workgroup and a grid
@@ -1127,24 +1210,20 @@ hybrid_pass_kernel(IoArgs io, CtlArgs c, HybridArgs h)
 {
     sct_table_init<K>();
     HybridCtl* ctl            = h.ctl;
-    const std::uint32_t par   = uniform(ctl->parity);
-    const std::uint32_t nbq   = uniform(ctl->nbatches);
+    const std::uint32_t par   = RG ? uniform(ctl->parity) : 0u;
+    const std::uint32_t nbq   = RG ? uniform(ctl->nbatches) : 0u;
     const std::uint32_t lane  = lane_id();
-    const std::uint32_t home  = blockIdx.x % kRanges;
 
-    // useful waves: queue batches plus input batches left
-    std::uint64_t left = 0;
-    for(std::uint32_t i = 0; i < kRanges; ++i)
-    {
-        const std::uint64_t nx = ctl->next[i].v, e = ctl->end[i].v;
-        left += nx < e ? (e - nx + 63) / 64 : 0;
-    }
-    left = uniform64(left);
-    if(std::uint64_t(blockIdx.x) >= nbq + left) return;
-    // drain pass: the input is exhausted and every queued batch has a wave
-    // of its own, so regrouping again cannot fill waves better than this
-    // pass does; survivors finish in place (no pass per remaining block)
-    const bool drain = left == 0 && nbq <= gridDim.x;
+    // a run without queues is one pass, so no counter is read before it claims
+    const Dealt         dealt(c.n, gridDim.x);
+    const std::uint32_t passes = RG ? uniform(ctl->passes) : 0u;
+    const std::uint32_t taken  = passes ? uniform(ctl->next[blockIdx.x % dealt.ranges].v) : 0u;
+    Reservoir res = deal(dealt, blockIdx.x, gridDim.x, passes == 0, taken);
+    if(passes && blockIdx.x >= nbq && res.chunk == 0) return;
+    // drain pass: the input was exhausted before it and every queued batch
+    // has a wave of its own, so regrouping again cannot fill waves better than
+    // this pass does; survivors finish in place (no pass per remaining block)
+    const bool drain = passes && nbq <= gridDim.x;
 
     [[maybe_unused]] const char*    qin  = h.q[par];
     [[maybe_unused]] char*          qout = h.q[par ^ 1u];
@@ -1153,7 +1232,6 @@ hybrid_pass_kernel(IoArgs io, CtlArgs c, HybridArgs h)
     WaveCtx w(c);
     std::uint64_t spill_rows = 0, spill_bytes = 0, fill_rows = 0, fill_bytes = 0,
                   admitted = 0, refills = 0, batches = 0, spill_failed = 0;
-    Reservoir res;
 
     RegsOf<K, CNT> r;
     std::uint32_t  pc  = HALT;
@@ -1192,18 +1270,16 @@ hybrid_pass_kernel(IoArgs io, CtlArgs c, HybridArgs h)
         }
         else
         {
-            std::uint64_t       base = 0;
-            const std::uint32_t got  = take_input(ctl, home, res, 64u, base);
-            if(!got) break;
-            if(lane < got)
+            const Taken t = take_input(ctl, dealt, c.n, res, 64u);
+            if(!t.count) break;
+            if(lane < t.count)
             {
-                const std::uint64_t t = base + lane;
-                load_inputs<K>(r, io.in, t);
-                tid = static_cast<std::uint32_t>(t);
+                tid = t.at(lane);
+                load_inputs<K>(r, io.in, tid);
                 pc  = 0;
                 has = true;
             }
-            admitted += got;
+            admitted += t.count;
         }
         ++batches;
 
@@ -1228,20 +1304,18 @@ hybrid_pass_kernel(IoArgs io, CtlArgs c, HybridArgs h)
             if(c.refill && ~live)
             {
                 const std::uint64_t empty = ~live;
-                std::uint64_t       base  = 0;
-                const std::uint32_t got   = take_input(ctl, home, res, popc(empty), base);
-                if(got)
+                const Taken t = take_input(ctl, dealt, c.n, res, popc(empty));
+                if(t.count)
                 {
                     const std::uint32_t k = rank_in(empty);
-                    if(!has && k < got)
+                    if(!has && k < t.count)
                     {
-                        const std::uint64_t t = base + k;
-                        load_inputs<K>(r, io.in, t);
-                        tid = static_cast<std::uint32_t>(t);
+                        tid = t.at(k);
+                        load_inputs<K>(r, io.in, tid);
                         pc  = 0;
                         has = true;
                     }
-                    admitted += got;
+                    admitted += t.count;
                     ++refills;
                     force = true;
                     continue;
@@ -1307,25 +1381,18 @@ hybrid_pass_kernel(IoArgs io, CtlArgs c, HybridArgs h)
 /// @p first set it initialises the control block.  One wave, lane 0 works.
 inline __global__ __launch_bounds__(64) void
 hybrid_setup_kernel(HybridCtl* ctl, std::uint32_t nb, std::uint64_t qcap,
-                    std::uint64_t n, std::uint32_t first)
+                    std::uint64_t n, std::uint32_t grid, std::uint32_t first)
 {
     if(threadIdx.x != 0) return;
     if(first)
     {
-        for(std::uint32_t r = 0; r < kRanges; ++r)
-        {
-            ctl->next[r].v = n * r / kRanges;
-            ctl->end[r].v  = n * (r + 1) / kRanges;
-        }
+        for(std::uint32_t r = 0; r < kRanges; ++r) ctl->next[r].v = 0;
         ctl->batch_next = 0;
         ctl->nbatches   = 0;
         ctl->parity     = 0;
         ctl->live       = 0;
         ctl->passes     = 0;
         ctl->done       = n == 0;
-        ctl->exhausted  = 0;
-        for(std::uint32_t r = 0; r < kRanges; ++r)
-            if(ctl->next[r].v >= ctl->end[r].v) ctl->exhausted |= 1u << r;
         for(int side = 0; side < 2; ++side)
             for(int l = 0; l < 64; ++l) ctl->qcount[side][l] = 0;
         for(int l = 0; l < 65; ++l) ctl->bprefix[l] = 0;
@@ -1344,15 +1411,14 @@ hybrid_setup_kernel(HybridCtl* ctl, std::uint32_t nb, std::uint64_t qcap,
     }
     ctl->bprefix[64] = pre;
     for(std::uint32_t l = 0; l < 64; ++l) ctl->qcount[out ^ 1u][l] = 0;
-    bool input_left = false;
-    std::uint32_t exhausted = 0;
-    for(std::uint32_t r = 0; r < kRanges; ++r)
+    bool        input_left = false;
+    const Dealt dealt(n, grid);
+    for(std::uint32_t r = 0; r < dealt.ranges; ++r)
     {
-        if(ctl->next[r].v > ctl->end[r].v) ctl->next[r].v = ctl->end[r].v;
-        input_left |= ctl->next[r].v < ctl->end[r].v;
-        if(ctl->next[r].v >= ctl->end[r].v) exhausted |= 1u << r;
+        const std::uint32_t total = dealt.claimed(r, grid);
+        if(ctl->next[r].v > total) ctl->next[r].v = total;
+        input_left |= ctl->next[r].v < total;
     }
-    ctl->exhausted  = exhausted;
     ctl->parity     = out;
     ctl->nbatches   = pre;
     ctl->batch_next = 0;

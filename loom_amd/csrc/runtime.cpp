@@ -228,7 +228,7 @@ run_hybrid_on(loom_context& x, const KernelEntry& e, const IoArgs& io, CtlArgs c
     const std::uint32_t nb = static_cast<std::uint32_t>(e.info.n_blocks);
     LOOM_HIP(hipEventRecord(x.ev[0], x.stream));
     hipLaunchKernelGGL(hybrid_setup_kernel, dim3(1), dim3(64), 0, x.stream, h.ctl, nb, h.qcap,
-                       c.n, 1u);
+                       c.n, grid, 1u);
     LOOM_HIP(hipGetLastError());
 
     std::uint32_t passes = 0, check_every = 1;
@@ -279,7 +279,7 @@ run_hybrid_on(loom_context& x, const KernelEntry& e, const IoArgs& io, CtlArgs c
                     evs.emplace_back(a, b);
                 }
                 hipLaunchKernelGGL(hybrid_setup_kernel, dim3(1), dim3(64), 0, x.stream, h.ctl, nb,
-                                   h.qcap, c.n, 0u);
+                                   h.qcap, c.n, grid, 0u);
                 LOOM_HIP(hipGetLastError());
                 ++passes;
             }
