@@ -67,9 +67,9 @@ claim_job_chunk(BatchCtl* ctl, const JobDesc* J, std::uint32_t j, std::uint32_t 
 
 /// @brief Run job @p j (kernel K) on this wave until the job has no more
 /// threads to admit and every lane halted.
-template <typename K, int P>
+template <typename K, int P, bool CNT>
 LOOM_DEVICE void
-run_job(const BatchArgs& a, std::uint32_t j, const CtlArgs& c, WaveCtx& w, std::uint64_t& admitted)
+run_job(const BatchArgs& a, std::uint32_t j, const CtlArgs& c, CtxOf<CNT>& w, std::uint64_t& admitted)
 {
     const JobDesc*      J   = a.jobs;
     const std::uint64_t len = J[j].end - J[j].begin;
@@ -81,11 +81,11 @@ run_job(const BatchArgs& a, std::uint32_t j, const CtlArgs& c, WaveCtx& w, std::
     std::uint32_t rcount = 0;
     bool          exhausted = false;
 
-    Regs<K>       r;
-    std::uint32_t pc  = HALT;
-    std::uint64_t tid = 0;
-    bool          has = false;
-    bool          force = true;
+    RegsOf<K, CNT> r;
+    std::uint32_t  pc  = HALT;
+    std::uint64_t  tid = 0;
+    bool           has = false;
+    bool           force = true;
 
     auto take = [&](std::uint32_t want, std::uint64_t& base) -> std::uint32_t
     {
@@ -103,7 +103,7 @@ run_job(const BatchArgs& a, std::uint32_t j, const CtlArgs& c, WaveCtx& w, std::
 
     for(;;)
     {
-        flush_if_high(w);
+        if constexpr(CNT) flush_if_high(w);
         const std::uint64_t live = ballot(has);
         if(~live)
         {
@@ -142,13 +142,14 @@ struct BatchSet
     static constexpr std::uint32_t size = sizeof...(Ks);
 };
 
-/// @brief The persistent batch kernel over the kernels @p Ks (policy @p P).
-template <int P, typename... Ks>
+/// @brief The persistent batch kernel over the kernels @p Ks (policy @p P;
+/// CNT: with work counts, else for runs that count none, see plain_run).
+template <int P, bool CNT, typename... Ks>
 __global__ __launch_bounds__(64) void
 batch_kernel(CtlArgs c, BatchArgs a)
 {
     (sct_table_init<Ks>(), ...);
-    WaveCtx w(c);
+    CtxOf<CNT> w(c);
     std::uint64_t admitted = 0;
     const std::uint32_t nj = a.njobs;
     // each wave walks the job list from its own start, so jobs of every size
@@ -165,13 +166,13 @@ batch_kernel(CtlArgs c, BatchArgs a)
         (
             [&]
             {
-                if(m == idx) run_job<Ks, P>(a, j, c, w, admitted);
+                if(m == idx) run_job<Ks, P, CNT>(a, j, c, w, admitted);
                 ++idx;
             }(),
             ...);
     }
     flush_stats(w);
-    if(c.stats && lane_id() == 0)
+    if(CNT && c.stats && lane_id() == 0)
         atomicAdd(&stat_slot(c)[ST_ADMITTED], static_cast<unsigned long long>(admitted));
     raise_errors(w.err, w.over, c);
 }

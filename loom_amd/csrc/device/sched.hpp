@@ -27,6 +27,7 @@
 #pragma once
 
 #include "memregs.hpp"
+#include "region.hpp"
 
 #include <hip/hip_runtime.h>
 
@@ -83,11 +84,14 @@ enum Stat : int
     ST_ACTIVE_FLOPS,   ///< Σ popcount(EXEC)·flops(B): useful floating-point work
 };
 
+/// @brief Dispatch budget of a run that sets none.
+inline constexpr std::uint64_t kDefaultSteps = 1ull << 40;
+
 /// @brief Per-run control arguments.
 struct CtlArgs
 {
     std::uint64_t  n         = 0;       ///< number of threads
-    std::uint64_t  max_steps = 1ull << 40; ///< per-wave block dispatch budget
+    std::uint64_t  max_steps = kDefaultSteps; ///< per-wave block dispatch budget
     std::uint32_t  thr       = 0;       ///< block-population threshold (lanes)
     std::uint32_t  live_thr  = 0;       ///< hybrid: stop when live lanes <= this
     std::uint32_t  refill    = 1;       ///< hybrid: refill free lanes in-wave
@@ -140,7 +144,7 @@ struct HybridArgs
 LOOM_DEVICE std::uint64_t
 ballot(bool p)
 {
-    return __ballot(p);
+    return __builtin_amdgcn_ballot_w64(p);
 }
 
 LOOM_DEVICE std::uint32_t
@@ -189,6 +193,8 @@ inline constexpr std::uint32_t kFlushSlots = 1u << 30;
 /// the sweep policy checks after every sweep, so the budget trips at most
 /// one sweep late.
 inline constexpr std::uint32_t kSegment = 128;
+/// Dispatches between checkpoints of a wave that counts no work.
+inline constexpr std::uint32_t kPlainSegment = 1u << 20;
 
 /// Blocks of at least this many ops count their work (thread steps, active
 /// operations and flops) from a scalar popcount of the block mask, on the
@@ -225,6 +231,27 @@ struct WaveCtx
     {
     }
 };
+
+/// @brief The state of a wave that counts no work (see plain_run): dispatches
+/// only, with nothing to flush and so with longer segments.
+struct PlainCtx : WaveCtx
+{
+    LOOM_DEVICE explicit PlainCtx(const CtlArgs& c) : WaveCtx(c)
+    {
+        stats = nullptr;
+        left  = static_cast<std::uint32_t>(rem < kPlainSegment ? rem : kPlainSegment);
+    }
+};
+
+/// @brief Run @p c counts no work: it collects no statistics, and its
+/// dispatch budget is the default one, so nothing depends on how dispatches
+/// are counted.  Kernels with small blocks are compiled for such runs a
+/// second time (Uncounted), where sweeps run whole regions.
+inline bool
+plain_run(const CtlArgs& c)
+{
+    return !c.stats && c.max_steps >= kDefaultSteps;
+}
 
 /// @brief This workgroup's copy of the counters.
 LOOM_DEVICE unsigned long long*
@@ -321,9 +348,20 @@ checkpoint(WaveCtx& w)
     w.left           = small ? static_cast<std::uint32_t>(w.rem) : kSegment;
 }
 
-/// @brief Checkpoint at the end of a segment (after a dispatch or a sweep).
 LOOM_DEVICE void
-segment_check(WaveCtx& w)
+checkpoint(PlainCtx& w)
+{
+    w.issued += w.disp;
+    w.over           = w.rem <= w.disp;
+    w.rem            = w.over ? 0 : w.rem - w.disp;
+    w.disp           = 0;
+    w.left           = static_cast<std::uint32_t>(w.rem < kPlainSegment ? w.rem : kPlainSegment);
+}
+
+/// @brief Checkpoint at the end of a segment (after a dispatch or a sweep).
+template <typename Ctx>
+LOOM_DEVICE void
+segment_check(Ctx& w)
 {
     if(__builtin_expect(w.disp >= w.left, 0)) checkpoint(w);
 }
@@ -334,22 +372,21 @@ segment_check(WaveCtx& w)
 inline constexpr std::uint32_t kMayHalt = 1u << 16;
 inline constexpr std::uint32_t kIndex   = 0xFFFFu;
 
-/// @brief The register file of a run that collects no statistics: small
-/// blocks then skip their per-lane work counts, which cost a kernel made of
-/// short blocks (Collatz's loop) about an eighth of its time.  Large blocks
-/// count on the scalar unit either way.
+/// @brief The register file of a run that counts no work (plain_run): its
+/// sweeps run the kernel's regions (region.hpp) instead of its blocks.
 template <typename K>
 struct Uncounted : Regs<K>
 {
 };
 
 template <typename RF>
-inline constexpr bool counts_small_blocks = true;
+inline constexpr bool sweeps_regions = false;
 template <typename K>
-inline constexpr bool counts_small_blocks<Uncounted<K>> = false;
+inline constexpr bool sweeps_regions<Uncounted<K>> = true;
 
-/// @brief Kernel @p K has a block below kScalarStepOps ops (only such
-/// kernels are compiled a second time without per-lane counts).
+/// @brief Kernel @p K has a block below kScalarStepOps ops.  Only such
+/// kernels are compiled a second time for runs that count no work: where
+/// every block is large, dispatching it costs little beside running it.
 template <typename K>
 inline constexpr bool has_small_blocks = []
 {
@@ -358,18 +395,27 @@ inline constexpr bool has_small_blocks = []
     return false;
 }();
 
-/// @brief The register file of kernel @p K's runs: counted, or not (CNT).
+/// @brief The register file and the wave state of kernel @p K's runs: counted,
+/// or not (CNT).
 template <typename K, bool CNT>
-using RegsOf = std::conditional_t<CNT, Regs<K>, Uncounted<K>>;
+using RegsOf = std::conditional_t<CNT || !has_small_blocks<K>, Regs<K>, Uncounted<K>>;
+template <bool CNT>
+using CtxOf = std::conditional_t<CNT, WaveCtx, PlainCtx>;
 
 /// @brief Run block @p B on the lanes at B and count the work.
-template <typename K, std::size_t B, typename RF>
+template <typename K, std::size_t B, typename RF, typename Ctx>
 LOOM_DEVICE void
-run_block(RF& r, std::uint32_t& pc, WaveCtx& w)
+run_block(RF& r, std::uint32_t& pc, Ctx& w)
 {
     constexpr ir::Block blk = ir::table_of<K>.block[B];
     static_assert(blk.flops <= 2u * blk.ops, "flops exceed twice the op count");
-    if constexpr(blk.ops >= kScalarStepOps)
+    w.disp += 1;
+    if constexpr(std::is_same_v<Ctx, PlainCtx>)
+    {
+        if(pc == B) exec_on<K, B>(r, pc, w.err);
+        return;
+    }
+    else if constexpr(blk.ops >= kScalarStepOps)
     {
         const std::uint32_t n = popc(ballot(pc == B));
         w.steps += n;
@@ -380,15 +426,11 @@ run_block(RF& r, std::uint32_t& pc, WaveCtx& w)
     else if(pc == B)
     {
         exec_on<K, B>(r, pc, w.err);
-        if constexpr(counts_small_blocks<RF>)
-        {
-            w.lane_steps += 1;
-            w.lane_ops += blk.ops;
-            if constexpr(blk.flops != 0) w.lane_flops += blk.flops;
-        }
+        w.lane_steps += 1;
+        w.lane_ops += blk.ops;
+        if constexpr(blk.flops != 0) w.lane_flops += blk.flops;
     }
     w.slots += 64u * blk.ops;
-    w.disp += 1;
 }
 
 /// @brief True when HALT is a successor of block @p B.
@@ -413,9 +455,9 @@ inline constexpr std::uint64_t halt_blocks = []
 
 /// @brief Run block @p B on the lanes at B and pick the next block among its
 /// successors (threaded dispatch, simd.hpp:3577-3731).
-template <typename K, std::size_t B, typename RF>
+template <typename K, std::size_t B, typename RF, typename Ctx>
 LOOM_DEVICE std::uint32_t
-step(RF& r, std::uint32_t& pc, std::uint64_t& pending, std::uint32_t thr, WaveCtx& w)
+step(RF& r, std::uint32_t& pc, std::uint64_t& pending, std::uint32_t thr, Ctx& w)
 {
     constexpr ir::Block blk = ir::table_of<K>.block[B];
 
@@ -464,10 +506,10 @@ step(RF& r, std::uint32_t& pc, std::uint64_t& pending, std::uint32_t thr, WaveCt
             return NONE;
 
 /// @brief Jump to the step of block @p cur (a wave-uniform value).
-template <typename K, typename RF>
+template <typename K, typename RF, typename Ctx>
 LOOM_DEVICE std::uint32_t
 dispatch(std::uint32_t cur, RF& r, std::uint32_t& pc, std::uint64_t& pending,
-         std::uint32_t thr, WaveCtx& w)
+         std::uint32_t thr, Ctx& w)
 {
     switch(cur)
     {
@@ -537,10 +579,10 @@ major_present(std::uint32_t pc, std::uint32_t& pops)
 /// runs regardless of the thresholds, which guarantees progress for every
 /// claimed batch.  Returns when no block has more than @p thr lanes (thr = 0:
 /// when every lane halted) or when at most @p live_thr lanes remain live.
-template <typename K, typename RF>
+template <typename K, typename RF, typename Ctx>
 LOOM_DEVICE void
 run_to_threshold(RF& r, std::uint32_t& pc, std::uint32_t thr, std::uint32_t live_thr,
-                 bool force, WaveCtx& w)
+                 bool force, Ctx& w)
 {
     std::uint64_t pending = 0;
     std::uint32_t pops    = 0;
@@ -665,9 +707,9 @@ topo_pick(std::uint64_t present)
 
 /// @brief POLICY_TOPO step: run the block of rank @p R, update the present
 /// set from its successors, pick the next rank.
-template <typename K, std::size_t R, typename RF>
+template <typename K, std::size_t R, typename RF, typename Ctx>
 LOOM_DEVICE std::uint32_t
-step_topo(RF& r, std::uint32_t& pc, std::uint64_t& present, WaveCtx& w)
+step_topo(RF& r, std::uint32_t& pc, std::uint64_t& present, Ctx& w)
 {
     constexpr std::size_t   B   = ir::table_of<K>.order[R];
     constexpr ir::Block     blk = ir::table_of<K>.block[B];
@@ -696,10 +738,10 @@ step_topo(RF& r, std::uint32_t& pc, std::uint64_t& present, WaveCtx& w)
         else                                                                              \
             return NONE;
 
-template <typename K, typename RF>
+template <typename K, typename RF, typename Ctx>
 LOOM_DEVICE std::uint32_t
 dispatch_topo(std::uint32_t cur, RF& r, std::uint32_t& pc, std::uint64_t& present,
-              WaveCtx& w)
+              Ctx& w)
 {
     switch(cur)
     {
@@ -723,9 +765,9 @@ dispatch_topo(std::uint32_t cur, RF& r, std::uint32_t& pc, std::uint64_t& presen
 
 /// @brief POLICY_TOPO runner: execute until every lane halted or at most
 /// @p live_thr lanes are live (the first step runs regardless with @p force).
-template <typename K, typename RF>
+template <typename K, typename RF, typename Ctx>
 LOOM_DEVICE void
-run_topo(RF& r, std::uint32_t& pc, std::uint32_t live_thr, bool force, WaveCtx& w)
+run_topo(RF& r, std::uint32_t& pc, std::uint32_t live_thr, bool force, Ctx& w)
 {
     std::uint64_t present = present_ranks<K>(pc);
     std::uint32_t cur     = topo_pick<K>(present);
@@ -741,12 +783,74 @@ run_topo(RF& r, std::uint32_t& pc, std::uint32_t live_thr, bool force, WaveCtx& 
     }
 }
 
+/// Trips of the loop of leader @p L between two looks at the wave: about 64
+/// operations, eight trips at most.  The look costs two vector and some ten
+/// scalar instructions; unrolled code costs registers and instruction cache.
+template <typename K, std::size_t L>
+inline constexpr int region_trips_of = []
+{
+    std::uint32_t ops = 0;
+    for(std::size_t b = 0; b < ir::table_of<K>.nb; ++b)
+        if(Regions<K>::map.of[b] == L) ops += ir::table_of<K>.block[b].ops;
+    return static_cast<int>(ops >= 64 ? 1 : (ops <= 8 ? 8 : 64 / ops));
+}();
+
+/// @brief Up to @p N trips of the loop of leader @p L on a lane at L.
+template <typename K, std::size_t L, int N>
+LOOM_DEVICE void
+region_trips(Regs<K>& r, std::uint32_t& pc, bool& in, std::uint32_t& err)
+{
+    std::uint32_t next = L;
+    exec_region<K, L>(r, next, err);
+    in = next == L;
+    if constexpr(Regions<K>::map.exit[L] == NONE) pc = next;
+    if constexpr(N > 1)
+        if(in) region_trips<K, L, N - 1>(r, pc, in, err);
+}
+
+/// @brief One region of a sweep that counts no work: run it on the lanes at
+/// its leader @p L and, if it is a loop that no other loop contains, again on
+/// those that came back to L, while more than @p live_thr did (the lanes that
+/// left it wait for the rest of the sweep; a wave that refills its free lanes
+/// does so below that).  Within the loop the lanes at L are a mask, not a
+/// program counter per lane; where all leave to the same place the counter is
+/// written once at the end.
+template <typename K, std::size_t L>
+LOOM_DEVICE void
+sweep_region(Regs<K>& r, std::uint32_t& pc, std::uint32_t live_thr, PlainCtx& w)
+{
+    using R                          = Regions<K>;
+    constexpr std::uint32_t blocks   = R::map.count[L];
+    constexpr bool          one_exit = R::map.exit[L] != NONE;
+    const bool              at       = pc == L;
+    if(!ballot(at)) return;
+    if constexpr(R::map.loops[L] && R::map.outer[L])
+    {
+        constexpr int trips = region_trips_of<K, L>;
+        bool          in    = at;
+        for(;;)
+        {
+            if(in) region_trips<K, L, trips>(r, pc, in, w.err);
+            w.disp += blocks * trips;
+            const std::uint32_t n = popc(ballot(in));
+            if(n <= live_thr || n == 0 || w.disp >= w.left) break;
+        }
+        if constexpr(one_exit)
+            if(at && !in) pc = LOOM_CX(R::map.exit[L]);
+    }
+    else
+    {
+        if(at) exec_region<K, L>(r, pc, w.err);
+        w.disp += blocks;
+    }
+}
+
 /// @brief POLICY_SWEEP runner: sweeps until every lane halted or, after a
 /// sweep, at most @p live_thr lanes are live (one sweep runs regardless when
 /// @p force is set).
-template <typename K, typename RF>
+template <typename K, typename RF, typename Ctx>
 LOOM_DEVICE void
-run_sweep(RF& r, std::uint32_t& pc, std::uint32_t live_thr, bool force, WaveCtx& w)
+run_sweep(RF& r, std::uint32_t& pc, std::uint32_t live_thr, bool force, Ctx& w)
 {
     if(!ballot(pc != HALT)) return;
     if(!force && live_thr && popc(ballot(pc != HALT)) <= live_thr) return;
@@ -758,7 +862,13 @@ run_sweep(RF& r, std::uint32_t& pc, std::uint32_t live_thr, bool force, WaveCtx&
                 [&]
                 {
                     constexpr std::size_t B = ir::table_of<K>.order[R];
-                    if(ballot(pc == B)) run_block<K, B>(r, pc, w);
+                    if constexpr(sweeps_regions<RF>)
+                    {
+                        if constexpr(Regions<K>::map.of[B] == B)
+                            sweep_region<K, B>(r, pc, live_thr, w);
+                    }
+                    else if(ballot(pc == B))
+                        run_block<K, B>(r, pc, w);
                 }(),
                 ...);
         }(std::make_index_sequence<ir::table_of<K>.nb>{});
@@ -771,10 +881,10 @@ run_sweep(RF& r, std::uint32_t& pc, std::uint32_t live_thr, bool force, WaveCtx&
 
 /// @brief Run the wave under policy @p P (see run_to_threshold / run_topo /
 /// run_sweep).
-template <typename K, int P, typename RF>
+template <typename K, int P, typename RF, typename Ctx>
 LOOM_DEVICE void
 run_policy(RF& r, std::uint32_t& pc, std::uint32_t thr, std::uint32_t live_thr, bool force,
-           WaveCtx& w)
+           Ctx& w)
 {
     if constexpr(P == POLICY_TOPO)
         run_topo<K>(r, pc, live_thr, force, w);
@@ -815,7 +925,7 @@ compact_kernel(IoArgs io, CtlArgs c)
         load_inputs<K>(r, io.in, tid);
         pc = 0;
     }
-    WaveCtx w(c);
+    CtxOf<CNT> w(c);
     run_policy<K, P>(r, pc, 0, 0, true, w);
     if(valid) store_outputs<K>(r, io.out, tid);
     flush_stats(w);
@@ -1229,7 +1339,7 @@ hybrid_pass_kernel(IoArgs io, CtlArgs c, HybridArgs h)
     [[maybe_unused]] char*          qout = h.q[par ^ 1u];
     [[maybe_unused]] std::uint32_t* qcnt = ctl->qcount[par ^ 1u];
 
-    WaveCtx w(c);
+    CtxOf<CNT> w(c);
     std::uint64_t spill_rows = 0, spill_bytes = 0, fill_rows = 0, fill_bytes = 0,
                   admitted = 0, refills = 0, batches = 0, spill_failed = 0;
 
@@ -1240,7 +1350,7 @@ hybrid_pass_kernel(IoArgs io, CtlArgs c, HybridArgs h)
 
     for(;;)
     {
-        flush_if_high(w);
+        if constexpr(CNT) flush_if_high(w);
         // ---- claim a batch (the wave is empty here) ----
         pc              = HALT;
         has             = false;
@@ -1360,7 +1470,7 @@ hybrid_pass_kernel(IoArgs io, CtlArgs c, HybridArgs h)
         if(w.over) break;
     }
     flush_stats(w);
-    if(c.stats && lane == 0)
+    if(CNT && c.stats && lane == 0)
     {
         auto* st = stat_slot(c);
         stat_add(st, ST_SPILL_ROWS, spill_rows);

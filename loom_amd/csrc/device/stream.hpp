@@ -122,7 +122,7 @@ store_state(const Regs<K>& r, const StreamArgs& a, std::uint64_t slot)
 /// most `live_thr` of them are live (or the dispatch budget of the step is
 /// spent: a step budget only ends the step, the threads keep their state),
 /// writes the registers back and appends the slots that halted to the ring.
-template <typename K, int P>
+template <typename K, int P, bool CNT = true>
 __global__ __launch_bounds__(64) void
 stream_step_kernel(StreamArgs a, CtlArgs c)
 {
@@ -131,14 +131,14 @@ stream_step_kernel(StreamArgs a, CtlArgs c)
     const std::uint32_t pc0  = a.pc[slot];
     const bool          live = pc0 < kHaltPc;
     if(!ballot(live)) return;
-    Regs<K>       r;
-    std::uint32_t pc = kHaltPc;
+    RegsOf<K, CNT> r;
+    std::uint32_t  pc = kHaltPc;
     if(live)
     {
         load_state<K>(r, a, slot);
         pc = pc0;
     }
-    WaveCtx w(c);
+    CtxOf<CNT> w(c);
     run_policy<K, P>(r, pc, c.thr, c.live_thr, true, w);
     if(live)
     {

@@ -236,7 +236,7 @@ wgr_kernel(IoArgs io, CtlArgs c, WgrArgs g)
     RegsOf<K, CNT>      r;
     std::uint32_t       pc  = HALT;
     std::uint32_t       tid = kNoTid;
-    WaveCtx             w(c);
+    CtxOf<CNT>          w(c);
     const std::uint64_t budget = c.max_steps ? c.max_steps : 1;
     bool                over   = false; // the run's dispatch budget is spent
     if(me == 0) s_stop = 0;
@@ -337,7 +337,9 @@ wgr_kernel(IoArgs io, CtlArgs c, WgrArgs g)
         w.issued += w.disp;
         w.disp = 0;
         w.rem  = g.phase ? g.phase : 1;
-        w.left = static_cast<std::uint32_t>(w.rem < kSegment ? w.rem : kSegment);
+        w.left = static_cast<std::uint32_t>(w.rem < (CNT ? kSegment : kPlainSegment) ?
+                                                w.rem :
+                                                (CNT ? kSegment : kPlainSegment));
         w.over = false;
         run_policy<K, P>(r, pc, c.thr, 0, true, w);
     }

@@ -83,7 +83,10 @@ template <int P, typename... Ks>
 hipError_t
 launch_batch(const CtlArgs& c, const BatchArgs& a, unsigned grid, hipStream_t s)
 {
-    hipLaunchKernelGGL((batch_kernel<P, Ks...>), dim3(grid), dim3(64), 0, s, c, a);
+    if(plain_run(c))
+        hipLaunchKernelGGL((batch_kernel<P, false, Ks...>), dim3(grid), dim3(64), 0, s, c, a);
+    else
+        hipLaunchKernelGGL((batch_kernel<P, true, Ks...>), dim3(grid), dim3(64), 0, s, c, a);
     return hipGetLastError();
 }
 
@@ -92,7 +95,7 @@ int
 batch_occupancy()
 {
     int nblk = 0;
-    if(hipOccupancyMaxActiveBlocksPerMultiprocessor(&nblk, batch_kernel<P, Ks...>, 64, 0) !=
+    if(hipOccupancyMaxActiveBlocksPerMultiprocessor(&nblk, batch_kernel<P, true, Ks...>, 64, 0) !=
        hipSuccess)
         return 1;
     return nblk > 0 ? nblk : 1;
@@ -122,11 +125,11 @@ launch_compact(const IoArgs& io, const CtlArgs& c, hipStream_t s)
 {
     if(c.n == 0) return hipSuccess;
     const std::uint64_t blocks = (c.n + 255) / 256;
-    // a run without statistics takes the kernel without per-lane work
-    // counts where the kernel has small blocks (the same kernel otherwise)
+    // a run that counts no work takes the kernel that sweeps regions where
+    // the kernel has small blocks (the same kernel otherwise)
     if constexpr(has_small_blocks<K>)
     {
-        if(!c.stats)
+        if(plain_run(c))
         {
             hipLaunchKernelGGL((compact_kernel<K, P, false>), dim3(static_cast<unsigned>(blocks)),
                                dim3(256), 0, s, io, c);
@@ -157,7 +160,7 @@ launch_wgr(const IoArgs& io, const CtlArgs& c, const WgrArgs& g, int waves, unsi
     if(c.n == 0) return hipSuccess;
     if constexpr(has_small_blocks<K>)
     {
-        if(!c.stats)
+        if(plain_run(c))
         {
             if(waves == 8)
                 hipLaunchKernelGGL((wgr_kernel<K, P, 8, false>), dim3(grid), dim3(64 * 8), 0, s, io,
@@ -190,9 +193,8 @@ wgr_occupancy(int waves)
 }
 
 /// Runs that regroup launch the pass kernel with the queue paths compiled
-/// in; the others the kernel without them, and those of them that collect
-/// no statistics, for a kernel with small blocks, the one without per-lane
-/// work counts.
+/// in; the others the kernel without them, and those of them that count no
+/// work, for a kernel with small blocks, the one that sweeps regions.
 template <typename K, int P>
 hipError_t
 launch_hybrid_pass(const IoArgs& io, const CtlArgs& c, const HybridArgs& h, unsigned grid,
@@ -200,7 +202,7 @@ launch_hybrid_pass(const IoArgs& io, const CtlArgs& c, const HybridArgs& h, unsi
 {
     if(c.regroup)
         hipLaunchKernelGGL((hybrid_pass_kernel<K, P, true>), dim3(grid), dim3(64), 0, s, io, c, h);
-    else if(has_small_blocks<K> && !c.stats)
+    else if(has_small_blocks<K> && plain_run(c))
         hipLaunchKernelGGL((hybrid_pass_kernel<K, P, false, !has_small_blocks<K>>), dim3(grid),
                            dim3(64), 0, s, io, c, h);
     else
@@ -267,8 +269,12 @@ hipError_t
 launch_stream_step(const StreamArgs& a, const CtlArgs& c, hipStream_t s)
 {
     if(a.slots == 0) return hipSuccess;
-    hipLaunchKernelGGL((stream_step_kernel<K, P>), dim3(static_cast<unsigned>(a.slots / 64)),
-                       dim3(64), 0, s, a, c);
+    if(has_small_blocks<K> && plain_run(c))
+        hipLaunchKernelGGL((stream_step_kernel<K, P, !has_small_blocks<K>>),
+                           dim3(static_cast<unsigned>(a.slots / 64)), dim3(64), 0, s, a, c);
+    else
+        hipLaunchKernelGGL((stream_step_kernel<K, P>), dim3(static_cast<unsigned>(a.slots / 64)),
+                           dim3(64), 0, s, a, c);
     return hipGetLastError();
 }
 

@@ -99,6 +99,50 @@ KERNEL(jump4, IVAR(i))
     IMOV(i, 11)
 KERNEL_END(IVAR(i));
 
+// A loop inside a loop, its body four ways (one of them straight back to the
+// inner loop's head, one out of both loops) with a join: every shape of
+// control flow that the other kernels leave out.
+template <std::unsigned_integral T>
+TKERNEL2(nested, a, b)
+    IBAND(n, a, 15),
+    IMOV(s, b),
+    IMOV(c, 0),
+    IEQ(f, n, 0),
+    IPJMP2(f, outer, HALT),
+    LABEL(outer),
+    IBAND(m, s, 7),
+    LABEL(inner),
+    IEQ(f, m, 0),
+    IPJMP2(f, work, tail),
+    LABEL(work),
+    IADD(c, c, 1),
+    IBAND(k, s, 3),
+    IPJMP4(k, add, mix, again, out),
+    LABEL(add),
+    IADD(s, s, n),
+    IADD(s, s, 1),
+    JMP(join),
+    LABEL(mix),
+    IMUL(s, s, 5),
+    IADD(s, s, m),
+    JMP(join),
+    LABEL(again),
+    IRSHFT(s, s, 1),
+    ISUB(m, m, 1),
+    JMP(inner),
+    LABEL(out),
+    IRSHFT(s, s, 2),
+    IBAND(f, s, 16),
+    IPJMP2(f, join, HALT),
+    LABEL(join),
+    ISUB(m, m, 1),
+    JMP(inner),
+    LABEL(tail),
+    ISUB(n, n, 1),
+    INEQ(f, n, 0),
+    IPJMP2(f, HALT, outer)
+TKERNEL_END2(s, c);
+
 // Integer op mix, straight-line: every binary integer operation of the
 // contract on (a, b), folded into several outputs.
 template <std::unsigned_integral T>
