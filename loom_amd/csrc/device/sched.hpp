@@ -1285,20 +1285,22 @@ LOOM_DEVICE Taken
 take_input(HybridCtl* ctl, const Dealt& d, std::uint64_t n, Reservoir& res, std::uint32_t want)
 {
     Taken t;
-    if(res.count == 0) next_batch(ctl, d, n, res);
-    t.base  = res.base;
-    t.head  = res.count < want ? res.count : want;
-    t.count = t.head;
-    res.base += t.head;
-    res.count -= t.head;
-    if(t.count < want && t.count != 0)
+    // a loop, so that the claim's code is there once
+#pragma unroll 1
+    for(int piece = 0; piece < 2; ++piece)
     {
-        next_batch(ctl, d, n, res);
+        if(res.count == 0) next_batch(ctl, d, n, res);
         const std::uint32_t g = res.count < want - t.count ? res.count : want - t.count;
         t.more                = res.base;
+        if(piece == 0)
+        {
+            t.base = res.base;
+            t.head = g;
+        }
         t.count += g;
         res.base += g;
         res.count -= g;
+        if(t.count == want || g == 0) break;
     }
     return t;
 }
@@ -1348,18 +1350,57 @@ hybrid_pass_kernel(IoArgs io, CtlArgs c, HybridArgs h)
     std::uint32_t  tid = 0;
     bool           has = false;
 
-    for(;;)
+    if constexpr(!RG)
     {
-        if constexpr(CNT) flush_if_high(w);
-        // ---- claim a batch (the wave is empty here) ----
-        pc              = HALT;
-        has             = false;
-        std::uint32_t b = nbq;
-        if(RG && lane == 0 && nbq) b = atomicAdd(&ctl->batch_next, 1u);
-        b = uniform(b);
-        if(RG && b < nbq)
+        // Without queues every wave takes input until none is left and then
+        // finishes its lanes in place.  One call site of the claim and one of
+        // the block code, which are inlined.
+        bool more = true;
+        for(;;)
         {
-            if constexpr(RG)
+            if constexpr(CNT) flush_if_high(w);
+            const std::uint64_t live = ballot(has);
+            bool                took = false;
+            if(more && ~live && (c.refill || !live))
+            {
+                const Taken t = take_input(ctl, dealt, c.n, res, popc(~live));
+                took          = t.count != 0;
+                more          = took;
+                if(took)
+                {
+                    const std::uint32_t k = rank_in(~live);
+                    if(!has && k < t.count)
+                    {
+                        tid = t.at(k);
+                        load_inputs<K>(r, io.in, tid);
+                        pc  = 0;
+                        has = true;
+                    }
+                    admitted += t.count;
+                    ++(live ? refills : batches);
+                }
+            }
+            if(!ballot(has)) break;
+            run_policy<K, P>(r, pc, took ? c.thr : 0u, took ? c.live_thr : 0u, true, w);
+            if(w.over) break;
+            if(has && pc == HALT)
+            {
+                store_outputs<K>(r, io.out, tid);
+                has = false;
+            }
+        }
+    }
+    else
+        for(;;)
+        {
+            if constexpr(CNT) flush_if_high(w);
+            // ---- claim a batch (the wave is empty here) ----
+            pc              = HALT;
+            has             = false;
+            std::uint32_t b = nbq;
+            if(lane == 0 && nbq) b = atomicAdd(&ctl->batch_next, 1u);
+            b = uniform(b);
+            if(b < nbq)
             {
                 // label of batch b: last label whose prefix is <= b
                 std::uint32_t label = 0;
@@ -1377,62 +1418,59 @@ hybrid_pass_kernel(IoArgs io, CtlArgs c, HybridArgs h)
                 fill_rows += rows;
                 fill_bytes += std::uint64_t(rows) * label_bytes<K>(label);
             }
-        }
-        else
-        {
-            const Taken t = take_input(ctl, dealt, c.n, res, 64u);
-            if(!t.count) break;
-            if(lane < t.count)
+            else
             {
-                tid = t.at(lane);
-                load_inputs<K>(r, io.in, tid);
-                pc  = 0;
-                has = true;
-            }
-            admitted += t.count;
-        }
-        ++batches;
-
-        // ---- execute, refill, spill ----
-        // One call site of the block code (it is inlined: a second site
-        // would double the kernel's instruction footprint).  `finish` runs
-        // the remaining lanes to HALT in place.
-        bool force = true, finish = false;
-        for(;;)
-        {
-            run_policy<K, P>(r, pc, finish ? 0u : c.thr, finish ? 0u : c.live_thr, force || finish,
-                             w);
-            force = false;
-            if(w.over) break;
-            if(has && pc == HALT)
-            {
-                store_outputs<K>(r, io.out, tid);
-                has = false;
-            }
-            const std::uint64_t live = ballot(has);
-            if(!live || finish) break;
-            if(c.refill && ~live)
-            {
-                const std::uint64_t empty = ~live;
-                const Taken t = take_input(ctl, dealt, c.n, res, popc(empty));
-                if(t.count)
+                const Taken t = take_input(ctl, dealt, c.n, res, 64u);
+                if(!t.count) break;
+                if(lane < t.count)
                 {
-                    const std::uint32_t k = rank_in(empty);
-                    if(!has && k < t.count)
-                    {
-                        tid = t.at(k);
-                        load_inputs<K>(r, io.in, tid);
-                        pc  = 0;
-                        has = true;
-                    }
-                    admitted += t.count;
-                    ++refills;
-                    force = true;
-                    continue;
+                    tid = t.at(lane);
+                    load_inputs<K>(r, io.in, tid);
+                    pc  = 0;
+                    has = true;
                 }
+                admitted += t.count;
             }
-            if constexpr(RG)
+            ++batches;
+
+            // ---- execute, refill, spill ----
+            // One call site of the block code (it is inlined: a second site
+            // would double the kernel's instruction footprint).  `finish` runs
+            // the remaining lanes to HALT in place.
+            bool force = true, finish = false;
+            for(;;)
             {
+                run_policy<K, P>(r, pc, finish ? 0u : c.thr, finish ? 0u : c.live_thr, force || finish,
+                                 w);
+                force = false;
+                if(w.over) break;
+                if(has && pc == HALT)
+                {
+                    store_outputs<K>(r, io.out, tid);
+                    has = false;
+                }
+                const std::uint64_t live = ballot(has);
+                if(!live || finish) break;
+                if(c.refill && ~live)
+                {
+                    const std::uint64_t empty = ~live;
+                    const Taken t = take_input(ctl, dealt, c.n, res, popc(empty));
+                    if(t.count)
+                    {
+                        const std::uint32_t k = rank_in(empty);
+                        if(!has && k < t.count)
+                        {
+                            tid = t.at(k);
+                            load_inputs<K>(r, io.in, tid);
+                            pc  = 0;
+                            has = true;
+                        }
+                        admitted += t.count;
+                        ++refills;
+                        force = true;
+                        continue;
+                    }
+                }
                 if(c.regroup && !drain)
                 {
                     // spill survivors into the queues of their labels
@@ -1463,12 +1501,11 @@ hybrid_pass_kernel(IoArgs io, CtlArgs c, HybridArgs h)
                     }
                     if(!ballot(has)) break;
                 }
+                // no regroup (or a full queue): finish the remaining lanes in place
+                finish = true;
             }
-            // no regroup (or a full queue): finish the remaining lanes in place
-            finish = true;
+            if(w.over) break;
         }
-        if(w.over) break;
-    }
     flush_stats(w);
     if(CNT && c.stats && lane == 0)
     {
