@@ -176,12 +176,4 @@ batch_kernel(CtlArgs c, BatchArgs a)
         atomicAdd(&stat_slot(c)[ST_ADMITTED], static_cast<unsigned long long>(admitted));
     raise_errors(w.err, w.over, c);
 }
-
-/// @brief Reset the claim cursors of a batch (one thread per job).
-inline __global__ void
-batch_reset_kernel(BatchArgs a)
-{
-    const std::uint32_t j = threadIdx.x;
-    if(j < a.njobs) a.ctl->next[j].v = a.jobs[j].begin;
-}
 } // namespace loom::hipvm

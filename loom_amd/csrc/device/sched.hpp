@@ -84,6 +84,12 @@ enum Stat : int
     ST_ACTIVE_FLOPS,   ///< Σ popcount(EXEC)·flops(B): useful floating-point work
 };
 
+/// Error flags (ErrorFlag) of a run: a word each, in pinned host memory, which
+/// a wave that raises one sets with a plain store.  The host clears them
+/// before the launch and reads them after it: a run that raises none costs no
+/// memset and no copy.
+inline constexpr std::uint32_t kErrWords = 3;
+
 /// @brief Dispatch budget of a run that sets none.
 inline constexpr std::uint64_t kDefaultSteps = 1ull << 40;
 
@@ -96,7 +102,7 @@ struct CtlArgs
     std::uint32_t  live_thr  = 0;       ///< hybrid: stop when live lanes <= this
     std::uint32_t  refill    = 1;       ///< hybrid: refill free lanes in-wave
     std::uint32_t  regroup   = 1;       ///< hybrid: spill survivors to queues
-    std::uint32_t* err       = nullptr; ///< error flags
+    std::uint32_t* err       = nullptr; ///< kErrWords words in host memory, one per error flag
     std::uint64_t* stats     = nullptr; ///< kStatSlots copies of kNumStats counters, or null
 };
 
@@ -113,14 +119,9 @@ struct alignas(256) Slot64
     std::uint64_t v;
 };
 
-struct alignas(256) Slot32
-{
-    std::uint32_t v;
-};
-
 struct HybridCtl
 {
-    Slot32        next[kRanges];  ///< batches claimed of each range
+    Slot64        next[kRanges];  ///< run << 32 | batches claimed of each range
     std::uint32_t batch_next;     ///< batch claim counter of the pass
     std::uint32_t nbatches;       ///< queue batches of the pass
     std::uint32_t parity;         ///< in-queue side of the pass
@@ -136,6 +137,9 @@ struct HybridArgs
     HybridCtl* ctl = nullptr;
     char*      q[2]{nullptr, nullptr}; ///< queue buffers (two sides)
     std::uint64_t qcap = 0;            ///< rows per label queue (multiple of 64)
+    /// number of the run on this control block: its cursors count from there
+    /// (claim_from).  0: a setup kernel cleared them.
+    std::uint32_t run = 0;
 };
 
 // ---------------------------------------------------------------------------
@@ -899,11 +903,9 @@ raise_errors(std::uint32_t lane_err, bool over, const CtlArgs& c)
 {
     std::uint32_t e = lane_err;
     if(over) e |= ERR_STEP_BUDGET;
-    // OR-reduce via ballots of each bit (few bits)
-    std::uint32_t we = 0;
-    for(std::uint32_t b = 0; b < 3; ++b)
-        if(ballot((e >> b) & 1u)) we |= 1u << b;
-    if(we && c.err && lane_id() == 0) atomicOr(c.err, we);
+    for(std::uint32_t b = 0; b < kErrWords; ++b)
+        if(ballot((e >> b) & 1u) && c.err && lane_id() == 0)
+            __hip_atomic_store(&c.err[b], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
 // ---------------------------------------------------------------------------
@@ -1233,10 +1235,29 @@ deal(const Dealt& d, std::uint32_t wave, std::uint32_t grid, bool first_pass, st
     return res;
 }
 
+/// @brief Add @p count to the cursor @p c of run @p run and return what it was:
+/// the upper bits (from @p Shift on) hold the number of the run that used it
+/// last, and the first waves to find an earlier run's there start it from 0
+/// (a maximum, which no wave that comes later can undo).  So no kernel has to
+/// clear the cursors between runs.
+template <int Shift>
+LOOM_DEVICE std::uint64_t
+claim_from(Slot64& c, std::uint64_t run, std::uint64_t count)
+{
+    auto*         p = reinterpret_cast<unsigned long long*>(&c.v);
+    std::uint64_t v = atomicAdd(p, static_cast<unsigned long long>(count));
+    if(v >> Shift != run)
+    {
+        atomicMax(p, static_cast<unsigned long long>(run << Shift));
+        v = atomicAdd(p, static_cast<unsigned long long>(count));
+    }
+    return v & ((std::uint64_t(1) << Shift) - 1u);
+}
+
 /// @brief Put the next batch in hand (claiming more when the reservoir holds
 /// none); count stays 0 once no input is left.
 LOOM_DEVICE void
-next_batch(HybridCtl* ctl, const Dealt& d, std::uint64_t n, Reservoir& res)
+next_batch(const HybridArgs& h, const Dealt& d, std::uint64_t n, Reservoir& res)
 {
     while(res.units == 0)
     {
@@ -1250,7 +1271,8 @@ next_batch(HybridCtl* ctl, const Dealt& d, std::uint64_t n, Reservoir& res)
         }
         const std::uint32_t total = d.claimed(res.range, gridDim.x);
         std::uint32_t       k     = 0;
-        if(lane_id() == 0) k = atomicAdd(&ctl->next[res.range].v, res.chunk);
+        if(lane_id() == 0)
+            k = static_cast<std::uint32_t>(claim_from<32>(h.ctl->next[res.range], h.run, res.chunk));
         k         = uniform(k);
         res.next  = d.rounds * gridDim.x + res.range + k * d.ranges;
         res.step  = d.ranges;
@@ -1282,14 +1304,14 @@ struct Taken
 };
 
 LOOM_DEVICE Taken
-take_input(HybridCtl* ctl, const Dealt& d, std::uint64_t n, Reservoir& res, std::uint32_t want)
+take_input(const HybridArgs& h, const Dealt& d, std::uint64_t n, Reservoir& res, std::uint32_t want)
 {
     Taken t;
     // a loop, so that the claim's code is there once
 #pragma unroll 1
     for(int piece = 0; piece < 2; ++piece)
     {
-        if(res.count == 0) next_batch(ctl, d, n, res);
+        if(res.count == 0) next_batch(h, d, n, res);
         const std::uint32_t g = res.count < want - t.count ? res.count : want - t.count;
         t.more                = res.base;
         if(piece == 0)
@@ -1321,7 +1343,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(RG ? regroup
 hybrid_pass_kernel(IoArgs io, CtlArgs c, HybridArgs h)
 {
     sct_table_init<K>();
-    HybridCtl* ctl            = h.ctl;
+    [[maybe_unused]] HybridCtl* ctl = h.ctl;
     const std::uint32_t par   = RG ? uniform(ctl->parity) : 0u;
     const std::uint32_t nbq   = RG ? uniform(ctl->nbatches) : 0u;
     const std::uint32_t lane  = lane_id();
@@ -1329,7 +1351,7 @@ hybrid_pass_kernel(IoArgs io, CtlArgs c, HybridArgs h)
     // a run without queues is one pass, so no counter is read before it claims
     const Dealt         dealt(c.n, gridDim.x);
     const std::uint32_t passes = RG ? uniform(ctl->passes) : 0u;
-    const std::uint32_t taken  = passes ? uniform(ctl->next[blockIdx.x % dealt.ranges].v) : 0u;
+    const std::uint32_t taken  = passes ? uniform(static_cast<std::uint32_t>(ctl->next[blockIdx.x % dealt.ranges].v)) : 0u;
     Reservoir res = deal(dealt, blockIdx.x, gridDim.x, passes == 0, taken);
     if(passes && blockIdx.x >= nbq && res.chunk == 0) return;
     // drain pass: the input was exhausted before it and every queued batch
@@ -1363,7 +1385,7 @@ hybrid_pass_kernel(IoArgs io, CtlArgs c, HybridArgs h)
             bool                took = false;
             if(more && ~live && (c.refill || !live))
             {
-                const Taken t = take_input(ctl, dealt, c.n, res, popc(~live));
+                const Taken t = take_input(h, dealt, c.n, res, popc(~live));
                 took          = t.count != 0;
                 more          = took;
                 if(took)
@@ -1420,7 +1442,7 @@ hybrid_pass_kernel(IoArgs io, CtlArgs c, HybridArgs h)
             }
             else
             {
-                const Taken t = take_input(ctl, dealt, c.n, res, 64u);
+                const Taken t = take_input(h, dealt, c.n, res, 64u);
                 if(!t.count) break;
                 if(lane < t.count)
                 {
@@ -1454,7 +1476,7 @@ hybrid_pass_kernel(IoArgs io, CtlArgs c, HybridArgs h)
                 if(c.refill && ~live)
                 {
                     const std::uint64_t empty = ~live;
-                    const Taken t = take_input(ctl, dealt, c.n, res, popc(empty));
+                    const Taken t = take_input(h, dealt, c.n, res, popc(empty));
                     if(t.count)
                     {
                         const std::uint32_t k = rank_in(empty);

@@ -49,9 +49,14 @@ inline constexpr std::size_t kWgrRoundWords = 31;
 /// workgroups per CU, so one runs while the other sorts).
 inline constexpr int kWgrWaves = 16;
 
+/// Bits of the input cursor below the run's number: 2^32 threads and the
+/// claims that find none left.
+inline constexpr int kWgrRunShift = 40;
+
 struct WgrArgs
 {
-    std::uint64_t* next  = nullptr; ///< input cursor (zero at launch)
+    Slot64*       next  = nullptr; ///< input cursor (claim_from, shifted by kWgrRunShift)
+    std::uint32_t run   = 0;       ///< number of the run on this cursor
     std::uint32_t  phase = 64;      ///< dispatch budget of a run phase
 };
 
@@ -239,6 +244,7 @@ wgr_kernel(IoArgs io, CtlArgs c, WgrArgs g)
     CtxOf<CNT>          w(c);
     const std::uint64_t budget = c.max_steps ? c.max_steps : 1;
     bool                over   = false; // the run's dispatch budget is spent
+    bool                dry    = false; // the input is exhausted (lane 0 of the workgroup)
     if(me == 0) s_stop = 0;
     __syncthreads();
     for(;;)
@@ -309,13 +315,13 @@ wgr_kernel(IoArgs io, CtlArgs c, WgrArgs g)
         {
             std::uint64_t base = 0;
             std::uint32_t got  = 0;
-            if(empty)
+            if(empty && !dry)
             {
-                base = atomicAdd(reinterpret_cast<unsigned long long*>(g.next),
-                                 static_cast<unsigned long long>(empty));
+                base = claim_from<kWgrRunShift>(*g.next, g.run, empty);
                 got  = base < c.n ? static_cast<std::uint32_t>(
                                        base + empty <= c.n ? empty : c.n - base) :
                                     0u;
+                dry  = got < empty;
             }
             s_got     = got;
             s_base_lo = static_cast<std::uint32_t>(base);

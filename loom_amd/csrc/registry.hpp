@@ -25,6 +25,14 @@
 
 namespace loom::hipvm
 {
+template <typename... P, typename... A>
+hipError_t
+launch(void (*kernel)(P...), std::uint64_t grid, unsigned block, hipStream_t s, const A&... args)
+{
+    hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(grid)), dim3(block), 0, s, P(args)...);
+    return hipGetLastError();
+}
+
 struct KernelEntry
 {
     loom_kernel_info info{};
@@ -40,7 +48,7 @@ struct KernelEntry
                          unsigned grid, hipStream_t) = {};
     int (*wgr_occupancy[2])(int waves) = {};
     hipError_t (*hybrid_pass[kNumPolicies])(const IoArgs&, const CtlArgs&, const HybridArgs&,
-                                 unsigned grid, hipStream_t)           = {};
+                                 unsigned grid, hipStream_t)       = {};
     /// resident 64-thread workgroups per CU of the hybrid pass kernel
     /// (with or without the regroup paths)
     int (*hybrid_occupancy[kNumPolicies])(bool regroup)                = {};
@@ -83,11 +91,8 @@ template <int P, typename... Ks>
 hipError_t
 launch_batch(const CtlArgs& c, const BatchArgs& a, unsigned grid, hipStream_t s)
 {
-    if(plain_run(c))
-        hipLaunchKernelGGL((batch_kernel<P, false, Ks...>), dim3(grid), dim3(64), 0, s, c, a);
-    else
-        hipLaunchKernelGGL((batch_kernel<P, true, Ks...>), dim3(grid), dim3(64), 0, s, c, a);
-    return hipGetLastError();
+    return plain_run(c) ? launch(batch_kernel<P, false, Ks...>, grid, 64, s, c, a) :
+                          launch(batch_kernel<P, true, Ks...>, grid, 64, s, c, a);
 }
 
 template <int P, typename... Ks>
@@ -128,17 +133,8 @@ launch_compact(const IoArgs& io, const CtlArgs& c, hipStream_t s)
     // a run that counts no work takes the kernel that sweeps regions where
     // the kernel has small blocks (the same kernel otherwise)
     if constexpr(has_small_blocks<K>)
-    {
-        if(plain_run(c))
-        {
-            hipLaunchKernelGGL((compact_kernel<K, P, false>), dim3(static_cast<unsigned>(blocks)),
-                               dim3(256), 0, s, io, c);
-            return hipGetLastError();
-        }
-    }
-    hipLaunchKernelGGL((compact_kernel<K, P>), dim3(static_cast<unsigned>(blocks)), dim3(256), 0, s,
-                       io, c);
-    return hipGetLastError();
+        if(plain_run(c)) return launch(compact_kernel<K, P, false>, blocks, 256, s, io, c);
+    return launch(compact_kernel<K, P>, blocks, 256, s, io, c);
 }
 
 template <typename K>
@@ -146,10 +142,7 @@ hipError_t
 launch_compact_mem(const IoArgs& io, const CtlArgs& c, const MemArgs& m, hipStream_t s)
 {
     if(c.n == 0) return hipSuccess;
-    const std::uint64_t blocks = (c.n + 255) / 256;
-    hipLaunchKernelGGL((compact_mem_kernel<K, POLICY_SWEEP>), dim3(static_cast<unsigned>(blocks)),
-                       dim3(256), 0, s, io, c, m);
-    return hipGetLastError();
+    return launch(compact_mem_kernel<K, POLICY_SWEEP>, (c.n + 255) / 256, 256, s, io, c, m);
 }
 
 template <typename K, int P>
@@ -159,23 +152,11 @@ launch_wgr(const IoArgs& io, const CtlArgs& c, const WgrArgs& g, int waves, unsi
 {
     if(c.n == 0) return hipSuccess;
     if constexpr(has_small_blocks<K>)
-    {
         if(plain_run(c))
-        {
-            if(waves == 8)
-                hipLaunchKernelGGL((wgr_kernel<K, P, 8, false>), dim3(grid), dim3(64 * 8), 0, s, io,
-                                   c, g);
-            else
-                hipLaunchKernelGGL((wgr_kernel<K, P, 16, false>), dim3(grid), dim3(64 * 16), 0, s,
-                                   io, c, g);
-            return hipGetLastError();
-        }
-    }
-    if(waves == 8)
-        hipLaunchKernelGGL((wgr_kernel<K, P, 8>), dim3(grid), dim3(64 * 8), 0, s, io, c, g);
-    else
-        hipLaunchKernelGGL((wgr_kernel<K, P, 16>), dim3(grid), dim3(64 * 16), 0, s, io, c, g);
-    return hipGetLastError();
+            return waves == 8 ? launch(wgr_kernel<K, P, 8, false>, grid, 64 * 8, s, io, c, g) :
+                                launch(wgr_kernel<K, P, 16, false>, grid, 64 * 16, s, io, c, g);
+    return waves == 8 ? launch(wgr_kernel<K, P, 8>, grid, 64 * 8, s, io, c, g) :
+                        launch(wgr_kernel<K, P, 16>, grid, 64 * 16, s, io, c, g);
 }
 
 template <typename K, int P>
@@ -200,14 +181,10 @@ hipError_t
 launch_hybrid_pass(const IoArgs& io, const CtlArgs& c, const HybridArgs& h, unsigned grid,
                    hipStream_t s)
 {
-    if(c.regroup)
-        hipLaunchKernelGGL((hybrid_pass_kernel<K, P, true>), dim3(grid), dim3(64), 0, s, io, c, h);
-    else if(has_small_blocks<K> && plain_run(c))
-        hipLaunchKernelGGL((hybrid_pass_kernel<K, P, false, !has_small_blocks<K>>), dim3(grid),
-                           dim3(64), 0, s, io, c, h);
-    else
-        hipLaunchKernelGGL((hybrid_pass_kernel<K, P, false>), dim3(grid), dim3(64), 0, s, io, c, h);
-    return hipGetLastError();
+    if(c.regroup) return launch(hybrid_pass_kernel<K, P, true>, grid, 64, s, io, c, h);
+    if(has_small_blocks<K> && plain_run(c))
+        return launch(hybrid_pass_kernel<K, P, false, !has_small_blocks<K>>, grid, 64, s, io, c, h);
+    return launch(hybrid_pass_kernel<K, P, false>, grid, 64, s, io, c, h);
 }
 
 template <typename K, int P>
@@ -270,12 +247,8 @@ launch_stream_step(const StreamArgs& a, const CtlArgs& c, hipStream_t s)
 {
     if(a.slots == 0) return hipSuccess;
     if(has_small_blocks<K> && plain_run(c))
-        hipLaunchKernelGGL((stream_step_kernel<K, P, !has_small_blocks<K>>),
-                           dim3(static_cast<unsigned>(a.slots / 64)), dim3(64), 0, s, a, c);
-    else
-        hipLaunchKernelGGL((stream_step_kernel<K, P>), dim3(static_cast<unsigned>(a.slots / 64)),
-                           dim3(64), 0, s, a, c);
-    return hipGetLastError();
+        return launch(stream_step_kernel<K, P, !has_small_blocks<K>>, a.slots / 64, 64, s, a, c);
+    return launch(stream_step_kernel<K, P>, a.slots / 64, 64, s, a, c);
 }
 
 template <typename K>

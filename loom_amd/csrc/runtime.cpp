@@ -94,9 +94,8 @@ context_init(loom_context& x)
     LOOM_HIP(hipSetDevice(g_dev.id));
     LOOM_HIP(hipStreamCreateWithFlags(&x.stream, hipStreamNonBlocking));
     LOOM_HIP(hipStreamCreateWithFlags(&x.copy, hipStreamNonBlocking));
-    LOOM_HIP(hipMalloc(&x.err, sizeof(std::uint32_t)));
+    LOOM_HIP(hipHostMalloc(&x.err, sizeof(std::uint32_t) * kErrWords, hipHostMallocDefault));
     LOOM_HIP(hipMalloc(&x.stats, sizeof(std::uint64_t) * kStatWords));
-    LOOM_HIP(hipHostMalloc(&x.host_err, sizeof(std::uint32_t), hipHostMallocDefault));
     LOOM_HIP(hipHostMalloc(&x.host_stats, sizeof(std::uint64_t) * kStatWords, hipHostMallocDefault));
     LOOM_HIP(hipHostMalloc(&x.host_ctl, sizeof(HybridCtl), hipHostMallocDefault));
     for(auto& ev: x.ev) LOOM_HIP(hipEventCreate(&ev));
@@ -120,36 +119,68 @@ context_release(loom_context& x)
     if(x.memregs) (void)hipFree(x.memregs);
     if(x.wgr_next) (void)hipFree(x.wgr_next);
     if(x.jobs) (void)hipFree(x.jobs);
+    if(x.host_jobs) (void)hipHostFree(x.host_jobs);
     if(x.bctl) (void)hipFree(x.bctl);
     for(auto& t: x.tickets) (void)hipEventDestroy(t.second);
     for(auto e: x.spare_events) (void)hipEventDestroy(e);
     for(auto e: x.pass_ev) (void)hipEventDestroy(e);
     for(auto e: x.ev)
         if(e) (void)hipEventDestroy(e);
-    if(x.err) (void)hipFree(x.err);
+    if(x.err) (void)hipHostFree(x.err);
     if(x.stats) (void)hipFree(x.stats);
-    if(x.host_err) (void)hipHostFree(x.host_err);
+    if(x.stage) (void)hipHostFree(x.stage);
     if(x.host_stats) (void)hipHostFree(x.host_stats);
     if(x.host_ctl) (void)hipHostFree(x.host_ctl);
     if(x.stream) (void)hipStreamDestroy(x.stream);
     if(x.copy) (void)hipStreamDestroy(x.copy);
 }
 
+/// @brief The flags and counters of a run whose kernels have finished.
 int
 finish_stats(loom_context& x, loom_run_stats* st, const loom_params* p)
 {
-    LOOM_HIP(hipMemcpyAsync(x.host_err, x.err, sizeof(std::uint32_t), hipMemcpyDeviceToHost,
-                            x.stream));
     if(p && p->collect_stats)
+    {
         LOOM_HIP(hipMemcpyAsync(x.host_stats, x.stats, sizeof(std::uint64_t) * kStatWords,
                                 hipMemcpyDeviceToHost, x.stream));
-    LOOM_HIP(hipStreamSynchronize(x.stream));
+        LOOM_HIP(hipStreamSynchronize(x.stream));
+        std::uint64_t sums[LOOM_NUM_COUNTERS]{};
+        sum_counters(x.host_stats, sums);
+        for(std::size_t i = 0; i < kNumStats; ++i)
+        {
+            if(st) st->counters[i] = sums[i] - x.stats_base[i];
+            x.stats_base[i] = sums[i];
+        }
+        x.stats_known = true;
+    }
+    const std::uint32_t e = error_flags(x.err);
+    if(st) st->errors = e;
+    if(e) return fail(LOOM_E_RUNTIME, "kernel raised error flags 0x%x", e);
+    return 0;
+}
+
+/// @brief A run that is one launch, made by @p f on @p x's stream: launch it
+/// between two events, wait for it and say how long it took.  (Events that
+/// take their times from the dispatch itself, hipExtLaunchKernel's, cost 8 us
+/// more per run than two records here.)
+template <typename F>
+int
+one_launch(loom_context& x, unsigned grid_waves, loom_run_stats* st, F&& f)
+{
+    LOOM_HIP(hipEventRecord(x.ev[0], x.stream));
+    LOOM_HIP(f());
+    LOOM_HIP(hipEventRecord(x.ev[1], x.stream));
+    LOOM_HIP(hipEventSynchronize(x.ev[1]));
+    float ms = 0;
+    LOOM_HIP(hipEventElapsedTime(&ms, x.ev[0], x.ev[1]));
     if(st)
     {
-        st->errors = *x.host_err;
-        if(p && p->collect_stats) sum_counters(x.host_stats, st->counters);
+        st->ms_total      = ms;
+        st->ms_main       = ms;
+        st->main_launches = 1;
+        st->passes        = 1;
+        st->grid_waves    = grid_waves;
     }
-    if(*x.host_err) return fail(LOOM_E_RUNTIME, "kernel raised error flags 0x%x", *x.host_err);
     return 0;
 }
 
@@ -175,24 +206,11 @@ run_compact(loom_context& x, const KernelEntry& e, const IoArgs& io, CtlArgs c, 
         m.base = x.memregs;
         m.rows = c.n;
     }
-    LOOM_HIP(hipEventRecord(x.ev[0], x.stream));
-    if(memory)
-        LOOM_HIP(e.compact_mem(io, c, m, x.stream));
-    else
-        LOOM_HIP(e.compact[policy](io, c, x.stream));
-    LOOM_HIP(hipEventRecord(x.ev[1], x.stream));
-    LOOM_HIP(hipEventSynchronize(x.ev[1]));
-    float ms = 0;
-    LOOM_HIP(hipEventElapsedTime(&ms, x.ev[0], x.ev[1]));
-    if(st)
-    {
-        st->ms_total      = ms;
-        st->ms_main       = ms;
-        st->main_launches = 1;
-        st->passes        = 1;
-        st->grid_waves    = static_cast<std::uint32_t>((c.n + 63) / 64);
-    }
-    return 0;
+    return one_launch(x, static_cast<unsigned>((c.n + 63) / 64), st,
+                      [&] {
+                          return memory ? e.compact_mem(io, c, m, x.stream) :
+                                          e.compact[policy](io, c, x.stream);
+                      });
 }
 
 /// @brief The persistent grid of a hybrid run: resident 64-lane workgroups
@@ -249,10 +267,8 @@ run_hybrid_on(loom_context& x, const KernelEntry& e, const IoArgs& io, CtlArgs c
     };
     if(!c.regroup)
     {
-        // One pass does all the work: every wave takes input until none is
-        // left and finishes its remaining lanes in place (a wave over its
-        // step budget raises the error flag instead), so no control-block
-        // read-back and host round trip is needed to learn that it is done.
+        // one pass does all the work (as in run_hybrid), so no control-block
+        // read-back and host round trip is needed to learn that it is done
         hipEvent_t a = next_ev(), b = next_ev();
         if(!a || !b) return fail(LOOM_E_RUNTIME, "event creation failed");
         LOOM_HIP(hipEventRecord(a, x.stream));
@@ -325,30 +341,22 @@ run_wgr(loom_context& x, const KernelEntry& e, const IoArgs& io, CtlArgs c, cons
 {
     const int which = p->reconv == POLICY_SUCCESSOR_MAJOR ? 0 : 1;
     const int waves = p->regroup_waves == 8 ? 8 : kWgrWaves;
-    if(!x.wgr_next) LOOM_HIP(hipMalloc(&x.wgr_next, sizeof(std::uint64_t)));
-    LOOM_HIP(hipMemsetAsync(x.wgr_next, 0, sizeof(std::uint64_t), x.stream));
+    if(!x.wgr_next) LOOM_HIP(hipMalloc(&x.wgr_next, sizeof(Slot64)));
+    if(x.wgr_run == 0 || x.wgr_run >= (1u << (64 - kWgrRunShift)) - 1u)
+    {
+        LOOM_HIP(hipMemsetAsync(x.wgr_next, 0, sizeof(Slot64), x.stream));
+        x.wgr_run = 0;
+    }
     WgrArgs g;
     g.next  = x.wgr_next;
+    g.run   = ++x.wgr_run;
     g.phase = p->regroup_phase ? p->regroup_phase : 64;
     const std::uint64_t lanes = 64ull * static_cast<std::uint64_t>(waves);
     const std::uint64_t need  = (c.n + lanes - 1) / lanes;
     unsigned grid = static_cast<unsigned>(g_dev.cus * e.wgr_occupancy[which](waves));
     if(need < grid) grid = static_cast<unsigned>(std::max<std::uint64_t>(1, need));
-    LOOM_HIP(hipEventRecord(x.ev[0], x.stream));
-    LOOM_HIP(e.wgr[which](io, c, g, waves, grid, x.stream));
-    LOOM_HIP(hipEventRecord(x.ev[1], x.stream));
-    LOOM_HIP(hipEventSynchronize(x.ev[1]));
-    float ms = 0;
-    LOOM_HIP(hipEventElapsedTime(&ms, x.ev[0], x.ev[1]));
-    if(st)
-    {
-        st->ms_total      = ms;
-        st->ms_main       = ms;
-        st->main_launches = 1;
-        st->passes        = 1;
-        st->grid_waves    = grid * static_cast<std::uint32_t>(waves);
-    }
-    return 0;
+    return one_launch(x, grid * static_cast<unsigned>(waves), st,
+                      [&] { return e.wgr[which](io, c, g, waves, grid, x.stream); });
 }
 
 int
@@ -365,6 +373,22 @@ run_hybrid(loom_context& x, int kidx, const KernelEntry& e, const IoArgs& io, Ct
     auto&             ws   = x.ws[kidx];
     const std::size_t side = std::size_t(qcap) * e.info.queue_row_bytes;
     if(!ws.ctl) LOOM_HIP(hipMalloc(&ws.ctl, sizeof(HybridCtl)));
+    if(!c.regroup && c.n)
+    {
+        // One launch: every wave takes input until none is left and finishes
+        // its remaining lanes in place (a wave over its step budget raises
+        // the error flag instead), and the cursors need no clearing, except
+        // when their run numbers begin or begin again.
+        if(ws.run == 0 || ws.run == 0xFFFFFFFFu)
+        {
+            LOOM_HIP(hipMemsetAsync(ws.ctl, 0, sizeof(HybridCtl), x.stream));
+            ws.run = 0;
+        }
+        HybridArgs h;
+        h.ctl = ws.ctl;
+        h.run = ++ws.run;
+        return one_launch(x, grid, st, [&] { return e.hybrid_pass[policy](io, c, h, grid, x.stream); });
+    }
     // queues are read only by runs that regroup
     if(c.regroup && ws.bytes < side)
     {
@@ -424,8 +448,14 @@ run_on(loom_context& x, int kernel, int mode, const void* const* inputs, void* c
     if(stats) *stats = loom_run_stats{};
     const IoArgs  io = n ? make_io(e, inputs, outputs) : IoArgs{};
     const CtlArgs c  = make_ctl(params, n, mode, x.err, x.stats);
-    LOOM_HIP(hipMemsetAsync(x.err, 0, sizeof(std::uint32_t), x.stream));
-    if(c.stats) LOOM_HIP(hipMemsetAsync(x.stats, 0, sizeof(std::uint64_t) * kStatWords, x.stream));
+    clear_errors(x.err);
+    if(c.stats)
+    {
+        if(!x.stats_known)
+            LOOM_HIP(hipMemsetAsync(x.stats, 0, sizeof(std::uint64_t) * kStatWords, x.stream));
+        if(!x.stats_known) std::fill(std::begin(x.stats_base), std::end(x.stats_base), 0);
+        x.stats_known = false;
+    }
     int r = 0;
     const bool memory = params && params->register_file == LOOM_REGFILE_MEMORY;
     if(memory && mode != LOOM_MODE_COMPACT)
@@ -444,6 +474,20 @@ run_on(loom_context& x, int kernel, int mode, const void* const* inputs, void* c
     return finish_stats(x, stats, params);
 }
 
+/// Host columns of a call that together take at most this much go through
+/// pinned memory that the kernel reads and writes itself: a copy costs about
+/// 15 us of queue and synchronisation per column, which reading over PCIe
+/// saves up to here (fib, 4099 threads, 64 KB: 107 us with copies, 67 without;
+/// 131,072 threads, 2 MB: 176 and 158; the cubic's 131,072, 6 MB: 344 and 410).
+constexpr std::size_t kStageBytes = std::size_t(2) << 20;
+
+/// @brief Bytes of a column of @p n elements, as a multiple of 256.
+std::size_t
+column_bytes(int type, std::uint64_t n)
+{
+    return (static_cast<std::size_t>(n) * type_size(type) + 255) / 256 * 256;
+}
+
 int
 run_host_on(loom_context& x, int kernel, int mode, const void* const* inputs,
             void* const* outputs, std::uint64_t n, const loom_params* params,
@@ -455,6 +499,25 @@ run_host_on(loom_context& x, int kernel, int mode, const void* const* inputs,
     if(int r = validate_run(e, mode, inputs, outputs, n, params)) return r;
     const int          ni = e.info.n_inputs, no = e.info.n_outputs;
     std::vector<void*> din(ni), dout(no);
+    std::size_t        total = 0;
+    for(int k = 0; k < ni + no; ++k)
+        total += column_bytes(k < ni ? e.info.input_type[k] : e.info.output_type[k - ni], n);
+    if(total <= kStageBytes)
+    {
+        if(!x.stage) LOOM_HIP(hipHostMalloc(&x.stage, kStageBytes, hipHostMallocDefault));
+        char* p = x.stage;
+        for(int k = 0; k < ni + no; ++k)
+        {
+            const int t                   = k < ni ? e.info.input_type[k] : e.info.output_type[k - ni];
+            (k < ni ? din[k] : dout[k - ni]) = p;
+            if(k < ni && n) std::memcpy(p, inputs[k], n * type_size(t));
+            p += column_bytes(t, n);
+        }
+        if(int r = run_on(x, kernel, mode, din.data(), dout.data(), n, params, stats)) return r;
+        for(int k = 0; k < no && n; ++k)
+            std::memcpy(outputs[k], dout[k], n * type_size(e.info.output_type[k]));
+        return 0;
+    }
     if(x.hostcol_ptr.size() < static_cast<std::size_t>(ni + no))
     {
         x.hostcol_ptr.resize(ni + no, nullptr);
@@ -507,12 +570,24 @@ launch_fill(void* dst, const void* pattern, std::uint64_t count, hipStream_t s)
     return hipGetLastError();
 }
 
-__global__ void
-zero_counters_kernel(std::uint32_t* err, std::uint64_t* stats, std::uint32_t nstats)
+/// @brief Before a batch launch, one workgroup per job: the job table from the
+/// host's pinned copy (if given) to the device's, the claim cursors, and zero
+/// for the counters (if the run collects them).
+__global__ __launch_bounds__(64) void
+batch_prepare_kernel(BatchArgs a, const JobDesc* host, JobDesc* table, std::uint64_t* stats)
 {
-    if(threadIdx.x == 0) *err = 0;
+    const std::uint32_t j = blockIdx.x;
+    if(host)
+    {
+        constexpr std::uint32_t words = sizeof(JobDesc) / sizeof(std::uint64_t);
+        const auto*             src   = reinterpret_cast<const std::uint64_t*>(host + j);
+        auto*                   dst   = reinterpret_cast<std::uint64_t*>(table + j);
+        for(std::uint32_t i = threadIdx.x; i < words; i += blockDim.x) dst[i] = src[i];
+    }
+    if(threadIdx.x == 0) a.ctl->next[j].v = host ? host[j].begin : a.jobs[j].begin;
     if(stats)
-        for(std::uint32_t i = threadIdx.x; i < nstats; i += blockDim.x) stats[i] = 0;
+        for(std::uint32_t i = j * blockDim.x + threadIdx.x; i < kStatWords; i += gridDim.x * blockDim.x)
+            stats[i] = 0;
 }
 
 int
@@ -584,9 +659,10 @@ batch_run_on(loom_context& x, int set, const loom_job* jobs, int njobs, const lo
     if(int r = batch_jobs(set, jobs, njobs, jd)) return r;
     if(stats) *stats = loom_run_stats{};
     if(!x.jobs) LOOM_HIP(hipMalloc(&x.jobs, sizeof(JobDesc) * kMaxJobs));
+    if(!x.host_jobs)
+        LOOM_HIP(hipHostMalloc(&x.host_jobs, sizeof(JobDesc) * kMaxJobs, hipHostMallocDefault));
     if(!x.bctl) LOOM_HIP(hipMalloc(&x.bctl, sizeof(BatchCtl)));
-    LOOM_HIP(hipMemcpyAsync(x.jobs, jd.data(), sizeof(JobDesc) * jd.size(), hipMemcpyHostToDevice,
-                            x.stream));
+    std::copy(jd.begin(), jd.end(), x.host_jobs); // no launch that reads it is in flight
     std::uint64_t threads = 0;
     for(const auto& j: jd) threads += j.end - j.begin;
     const BatchEntry& b = batch_registry()[set];
@@ -596,24 +672,13 @@ batch_run_on(loom_context& x, int set, const loom_job* jobs, int njobs, const lo
     a.ctl   = x.bctl;
     a.njobs = static_cast<std::uint32_t>(njobs);
     const unsigned grid = batch_grid(b, params, threads);
-    hipLaunchKernelGGL(zero_counters_kernel, dim3(1), dim3(64), 0, x.stream, x.err, x.stats,
-                       static_cast<std::uint32_t>(kStatWords));
-    hipLaunchKernelGGL(batch_reset_kernel, dim3(1), dim3(kMaxJobs), 0, x.stream, a);
-    LOOM_HIP(hipGetLastError());
-    LOOM_HIP(hipEventRecord(x.ev[0], x.stream));
-    LOOM_HIP(b.launch[batch_policy(params)](c, a, grid, x.stream));
-    LOOM_HIP(hipEventRecord(x.ev[1], x.stream));
-    LOOM_HIP(hipEventSynchronize(x.ev[1]));
-    float ms = 0;
-    LOOM_HIP(hipEventElapsedTime(&ms, x.ev[0], x.ev[1]));
-    if(stats)
-    {
-        stats->ms_total      = ms;
-        stats->ms_main       = ms;
-        stats->main_launches = 1;
-        stats->passes        = 1;
-        stats->grid_waves    = grid;
-    }
+    clear_errors(x.err);
+    x.stats_known = false;
+    LOOM_HIP(launch(batch_prepare_kernel, njobs, 64, x.stream, a, x.host_jobs, x.jobs, c.stats));
+    if(c.stats) std::fill(std::begin(x.stats_base), std::end(x.stats_base), 0);
+    if(int r = one_launch(x, grid, stats,
+                          [&] { return b.launch[batch_policy(params)](c, a, grid, x.stream); }))
+        return r;
     return finish_stats(x, stats, params);
 }
 
@@ -1326,14 +1391,14 @@ loom_batch_graph_create(int set, const loom_job* jobs, int njobs, const loom_par
     g->grid = batch_grid(b, params, threads);
     // counters are cleared by a kernel node (no memset nodes in the graph)
     LOOM_HIP(hipStreamBeginCapture(x.stream, hipStreamCaptureModeThreadLocal));
-    hipLaunchKernelGGL(zero_counters_kernel, dim3(1), dim3(64), 0, x.stream, x.err, x.stats,
-                       static_cast<std::uint32_t>(kStatWords));
-    hipLaunchKernelGGL(batch_reset_kernel, dim3(1), dim3(kMaxJobs), 0, x.stream, a);
+    const hipError_t pe = launch(batch_prepare_kernel, njobs, 64, x.stream, a,
+                                 static_cast<const JobDesc*>(nullptr),
+                                 static_cast<JobDesc*>(nullptr), c.stats);
     const hipError_t le = b.launch[batch_policy(params)](c, a, g->grid, x.stream);
     const hipError_t ce = hipStreamEndCapture(x.stream, &g->graph);
-    if(le != hipSuccess || ce != hipSuccess)
-        return fail(LOOM_E_RUNTIME, "graph capture failed: %s",
-                    hipGetErrorString(le != hipSuccess ? le : ce));
+    for(const hipError_t e: {pe, le, ce})
+        if(e != hipSuccess)
+            return fail(LOOM_E_RUNTIME, "graph capture failed: %s", hipGetErrorString(e));
     LOOM_HIP(hipGraphInstantiate(&g->exec, g->graph, nullptr, nullptr, 0));
     *graph = g.release();
     return 0;
@@ -1347,20 +1412,11 @@ loom_graph_launch(loom_graph* g, loom_run_stats* stats)
     if(int r = lock_context(g->ctx, l)) return r;
     loom_context& x = *l.x;
     if(stats) *stats = loom_run_stats{};
-    LOOM_HIP(hipEventRecord(x.ev[0], x.stream));
-    LOOM_HIP(hipGraphLaunch(g->exec, x.stream));
-    LOOM_HIP(hipEventRecord(x.ev[1], x.stream));
-    LOOM_HIP(hipEventSynchronize(x.ev[1]));
-    float ms = 0;
-    LOOM_HIP(hipEventElapsedTime(&ms, x.ev[0], x.ev[1]));
-    if(stats)
-    {
-        stats->ms_total      = ms;
-        stats->ms_main       = ms;
-        stats->main_launches = 1;
-        stats->passes        = 1;
-        stats->grid_waves    = g->grid;
-    }
+    clear_errors(x.err);
+    x.stats_known = false;
+    std::fill(std::begin(x.stats_base), std::end(x.stats_base), 0);
+    if(int r = one_launch(x, g->grid, stats, [&] { return hipGraphLaunch(g->exec, x.stream); }))
+        return r;
     return finish_stats(x, stats, g->has_params ? &g->params : nullptr);
 }
 

@@ -57,6 +57,22 @@ int validate_params(const loom_params* params);
 CtlArgs make_ctl(const loom_params* p, std::uint64_t n, int mode, std::uint32_t* err,
                  std::uint64_t* stats);
 
+/// @brief Clear the error words of a run before its launch (no kernel that
+/// could write them is in flight then), and their flags after it.
+inline void
+clear_errors(std::uint32_t* words)
+{
+    for(std::uint32_t b = 0; b < kErrWords; ++b) __atomic_store_n(&words[b], 0u, __ATOMIC_RELEASE);
+}
+inline std::uint32_t
+error_flags(const std::uint32_t* words)
+{
+    std::uint32_t e = 0;
+    for(std::uint32_t b = 0; b < kErrWords; ++b)
+        if(__atomic_load_n(&words[b], __ATOMIC_ACQUIRE)) e |= 1u << b;
+    return e;
+}
+
 /// @brief Sum the counter copies of a run into @p out.
 void sum_counters(const std::uint64_t* host_stats, std::uint64_t* out);
 } // namespace loom::hipvm
@@ -71,14 +87,18 @@ struct loom_context
     std::mutex     mu;
     hipStream_t    stream{};
     hipStream_t    copy{};
-    std::uint32_t* err        = nullptr; ///< device error flags
+    std::uint32_t* err        = nullptr; ///< error words (pinned, written by kernels)
     std::uint64_t* stats      = nullptr; ///< device counters (kStatWords)
-    std::uint32_t* host_err   = nullptr; ///< pinned
     std::uint64_t* host_stats = nullptr; ///< pinned
+    /// sums of `stats` that earlier runs left there, which are not cleared but
+    /// subtracted; false while a run may have added to them unread
+    std::uint64_t  stats_base[loom::hipvm::kNumStats]{};
+    bool           stats_known = false;
     loom::hipvm::HybridCtl* host_ctl = nullptr; ///< pinned mirror of a control block
     hipEvent_t     ev[4]{};
     std::vector<hipEvent_t> pass_ev;
     loom::hipvm::JobDesc*  jobs = nullptr; ///< device job table of direct batch runs
+    loom::hipvm::JobDesc*  host_jobs = nullptr; ///< pinned: the table as the host wrote it
     loom::hipvm::BatchCtl* bctl = nullptr;
     /// background copies: tickets of outstanding copies, oldest first
     std::deque<std::pair<std::uint64_t, hipEvent_t>> tickets;
@@ -90,11 +110,16 @@ struct loom_context
         loom::hipvm::HybridCtl* ctl   = nullptr;
         char*                   q[2]  = {nullptr, nullptr};
         std::size_t             bytes = 0; ///< per side
+        std::uint32_t           run   = 0; ///< runs on ctl's cursors (claim_from)
     };
     std::vector<Workspace> ws; ///< per kernel index
 
-    /// input cursor of workgroup-regrouping runs
-    std::uint64_t* wgr_next = nullptr;
+    /// input cursor of workgroup-regrouping runs, and its runs
+    loom::hipvm::Slot64* wgr_next = nullptr;
+    std::uint32_t        wgr_run  = 0;
+
+    /// pinned columns of small loom_run_host calls
+    char* stage = nullptr;
 
     /// register file of compact runs in device memory, grown on demand
     char*       memregs       = nullptr;

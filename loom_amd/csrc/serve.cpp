@@ -233,6 +233,9 @@ serve(loom_server* s, Source& src, clock_type::time_point t0, loom_server_stats*
 {
     loom_context*     ctx = s->ctx;
     loom_server_stats st{};
+    // nobody reads the counters of a step: its launches need not count
+    loom_params params   = s->cfg.params;
+    params.collect_stats = 0;
     auto now = [&] { return std::chrono::duration<double, std::milli>(clock_type::now() - t0).count(); };
 
     // kernel infos: every registered kernel can be served; members of the
@@ -480,7 +483,7 @@ serve(loom_server* s, Source& src, clock_type::time_point t0, loom_server_stats*
         if(!jobs.empty())
         {
             if(int e = loom_ctx_batch_run(ctx, s->cfg.batch_set, jobs.data(),
-                                          static_cast<int>(jobs.size()), &s->cfg.params, &rs))
+                                          static_cast<int>(jobs.size()), &params, &rs))
             {
                 for(auto& r: running) r.req->status = e;
                 return fail(e);
@@ -503,7 +506,7 @@ serve(loom_server* s, Source& src, clock_type::time_point t0, loom_server_stats*
                 outs[k] = running[i].out[k] + b * type_bytes(ki.output_type[k]);
             loom_run_stats ks{};
             if(int e = loom_ctx_run(ctx, q.kernel, LOOM_MODE_HYBRID, ins, outs, ends[i] - b,
-                                    &s->cfg.params, &ks))
+                                    &params, &ks))
             {
                 for(auto& r: running) r.req->status = e;
                 return fail(e);

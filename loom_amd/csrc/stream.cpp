@@ -43,9 +43,8 @@ struct loom_stream
     /// staging columns (device) of inputs in and outputs out, S rows each
     std::vector<char*> in_stage, out_stage;
     std::uint64_t*     ids_stage = nullptr;
-    std::uint32_t*     err       = nullptr;
+    std::uint32_t*     err       = nullptr; ///< error words (pinned, written by kernels)
     std::uint64_t*     stats     = nullptr;
-    std::uint32_t*     host_err  = nullptr; ///< pinned
     std::uint64_t*     host_stats = nullptr; ///< pinned
     hipEvent_t         ev[2]{};
     /// host view of the stream (exact after every call)
@@ -59,15 +58,14 @@ struct loom_stream
         if(stream) (void)hipStreamSynchronize(stream);
         for(void* p: {static_cast<void*>(regs), static_cast<void*>(pc), static_cast<void*>(tid),
                       static_cast<void*>(ring), static_cast<void*>(ctl),
-                      static_cast<void*>(ids_stage), static_cast<void*>(err),
-                      static_cast<void*>(stats)})
+                      static_cast<void*>(ids_stage), static_cast<void*>(stats)})
             if(p) (void)hipFree(p);
         for(char* p: in_stage)
             if(p) (void)hipFree(p);
         for(char* p: out_stage)
             if(p) (void)hipFree(p);
         if(host_ctl) (void)hipHostFree(host_ctl);
-        if(host_err) (void)hipHostFree(host_err);
+        if(err) (void)hipHostFree(err);
         if(host_stats) (void)hipHostFree(host_stats);
         for(auto ev: this->ev)
             if(ev) (void)hipEventDestroy(ev);
@@ -170,10 +168,9 @@ loom_stream_create(int kernel, uint64_t slots, const loom_params* params, loom_s
     LOOM_HIP(hipMalloc(&s->ring, slots * sizeof(std::uint32_t)));
     LOOM_HIP(hipMalloc(&s->ctl, sizeof(StreamCtl)));
     LOOM_HIP(hipMalloc(&s->ids_stage, slots * sizeof(std::uint64_t)));
-    LOOM_HIP(hipMalloc(&s->err, sizeof(std::uint32_t)));
+    LOOM_HIP(hipHostMalloc(&s->err, sizeof(std::uint32_t) * kErrWords, hipHostMallocDefault));
     LOOM_HIP(hipMalloc(&s->stats, sizeof(std::uint64_t) * kStatWords));
     LOOM_HIP(hipHostMalloc(&s->host_ctl, sizeof(StreamCtl), hipHostMallocDefault));
-    LOOM_HIP(hipHostMalloc(&s->host_err, sizeof(std::uint32_t), hipHostMallocDefault));
     LOOM_HIP(hipHostMalloc(&s->host_stats, sizeof(std::uint64_t) * kStatWords, hipHostMallocDefault));
     for(auto& ev: s->ev) LOOM_HIP(hipEventCreate(&ev));
     for(int k = 0; k < s->e->info.n_inputs; ++k)
@@ -239,14 +236,12 @@ loom_stream_step(loom_stream* s, loom_run_stats* stats)
     if(stats) *stats = loom_run_stats{};
     const loom_params& p = s->params;
     CtlArgs            c = make_ctl(&p, s->live, LOOM_MODE_HYBRID, s->err, s->stats);
-    LOOM_HIP(hipMemsetAsync(s->err, 0, sizeof(std::uint32_t), s->stream));
+    clear_errors(s->err);
     if(c.stats) LOOM_HIP(hipMemsetAsync(s->stats, 0, sizeof(std::uint64_t) * kStatWords, s->stream));
     LOOM_HIP(hipEventRecord(s->ev[0], s->stream));
     if(s->live) LOOM_HIP(s->e->stream_step[p.reconv](s->a, c, s->stream));
     LOOM_HIP(hipEventRecord(s->ev[1], s->stream));
     LOOM_HIP(hipMemcpyAsync(s->host_ctl, s->ctl, sizeof(StreamCtl), hipMemcpyDeviceToHost, s->stream));
-    LOOM_HIP(hipMemcpyAsync(s->host_err, s->err, sizeof(std::uint32_t), hipMemcpyDeviceToHost,
-                            s->stream));
     if(c.stats)
         LOOM_HIP(hipMemcpyAsync(s->host_stats, s->stats, sizeof(std::uint64_t) * kStatWords,
                                 hipMemcpyDeviceToHost, s->stream));
@@ -257,6 +252,7 @@ loom_stream_step(loom_stream* s, loom_run_stats* stats)
     ++s->counters.steps;
     float ms = 0;
     LOOM_HIP(hipEventElapsedTime(&ms, s->ev[0], s->ev[1]));
+    const std::uint32_t e = error_flags(s->err);
     if(stats)
     {
         stats->ms_total      = ms;
@@ -264,10 +260,10 @@ loom_stream_step(loom_stream* s, loom_run_stats* stats)
         stats->main_launches = 1;
         stats->passes        = 1;
         stats->grid_waves    = static_cast<std::uint32_t>(s->slots / 64);
-        stats->errors        = *s->host_err;
+        stats->errors        = e;
         if(c.stats) sum_counters(s->host_stats, stats->counters);
     }
-    if(*s->host_err) return fail(LOOM_E_RUNTIME, "kernel raised error flags 0x%x", *s->host_err);
+    if(e) return fail(LOOM_E_RUNTIME, "kernel raised error flags 0x%x", e);
     return 0;
 }
 
