@@ -35,7 +35,7 @@ DEFAULT = {"live_threshold": 48, "regroup": False, "reconv": 2, "waves_per_cu": 
 
 SPACE = {
     # 0: refill only once every lane of the wave halted
-    "live_threshold": [0, 32, 40, 48, 56],
+    "live_threshold": [0, 32, 48, 56, 60],
     "regroup": [False, True],
     "reconv": [0, 1, 2],
     "waves_per_cu": [0, 8, 16, 20],
@@ -148,7 +148,7 @@ def tune(kernel_name: str, inputs, reps: int = 2, space: dict | None = None,
 
 
 BATCH_SPACE = {
-    "live_threshold": [0, 32, 48, 56],
+    "live_threshold": [0, 48, 56, 60],
     "waves_per_cu": [0, 12, 16],
     "reconv": [1, 2],
 }

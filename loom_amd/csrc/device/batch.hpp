@@ -81,56 +81,36 @@ run_job(const BatchArgs& a, std::uint32_t j, const CtlArgs& c, CtxOf<CNT>& w, st
     std::uint32_t rcount = 0;
     bool          exhausted = false;
 
-    RegsOf<K, CNT> r;
-    std::uint32_t  pc  = HALT;
-    std::uint64_t  tid = 0;
-    bool           has = false;
-    bool           force = true;
+    Lanes<K, P, RegsOf<K, CNT>> l;
+    bool                        force = true;
 
-    auto take = [&](std::uint32_t want, std::uint64_t& base) -> std::uint32_t
+    auto input = [&](std::uint32_t want)
     {
         if(rcount == 0 && !exhausted)
         {
-            rcount = claim_job_chunk(a.ctl, J, j, chunk, rbase);
-            if(!rcount) exhausted = true;
+            rcount    = claim_job_chunk(a.ctl, J, j, chunk, rbase);
+            exhausted = rcount == 0;
         }
-        const std::uint32_t g = rcount < want ? rcount : want;
-        base                  = rbase;
-        rbase += g;
-        rcount -= g;
-        return g;
+        Taken t;
+        t.count = t.head = rcount < want ? rcount : want;
+        t.base           = static_cast<std::uint32_t>(rbase);
+        rbase += t.count;
+        rcount -= t.count;
+        return t;
     };
 
     for(;;)
     {
         if constexpr(CNT) flush_if_high(w);
-        const std::uint64_t live = ballot(has);
-        if(~live)
-        {
-            std::uint64_t       base = 0;
-            const std::uint64_t empty = ~live;
-            const std::uint32_t got   = take(popc(empty), base);
-            if(got)
-            {
-                const std::uint32_t k = rank_in(empty);
-                if(!has && k < got)
-                {
-                    tid = base + k;
-                    load_inputs<K>(r, J[j].in, tid);
-                    pc  = 0;
-                    has = true;
-                }
-                admitted += got;
-                force = true;
-            }
-        }
-        if(!ballot(has)) return;
-        run_policy<K, P>(r, pc, 0, exhausted ? 0u : c.live_thr, force, w);
+        const std::uint64_t live = ballot(l.has);
+        if(~live && l.input_left() && l.refill(~live, J[j], w, input, admitted)) force = true;
+        if(!ballot(l.has)) return;
+        run_policy<K, P, l.pooled>(l.r, l.pc, 0, l.input_left() ? c.live_thr : 0u, force, w);
         force = false;
-        if(has && pc == HALT)
+        if(l.has && l.pc == HALT)
         {
-            store_outputs<K>(r, J[j].out, tid);
-            has = false;
+            store_outputs<K>(l.r, J[j].out, l.tid);
+            l.has = false;
         }
         if(w.over) return;
     }

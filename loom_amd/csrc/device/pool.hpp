@@ -1,0 +1,151 @@
+// -*- C++ -*-
+/// @file pool.hpp
+/// @brief A wave's pool of started threads, in LDS.
+///
+/// A wave that refills its free lanes runs START on those lanes alone: the
+/// path tracer's START is a quarter of a bounce's instructions and ran on 16
+/// of 64 lanes, which also kept the refill threshold low (48).  With a pool
+/// START runs on 64 new threads at once; what is live after it (the registers
+/// live into its successors, the thread id, the next block if there are
+/// several) waits in LDS, one column of 64 words each, and a refill reads it
+/// from there.  Registers that START sets to a literal are set again at the
+/// refill instead.  Threads that halt in START never enter the pool.
+///
+/// The path tracer's 1024x768x64 frame: 7.24 ms without the pool (refilled at 48
+/// lanes, 72% of the lanes active), 6.44 with it (refilled at 60, 81%).
+///
+/// Used where it pays: START of at least kPoolMinOps operations that no other
+/// block jumps back to, in waves that own their workgroup's LDS.
+#pragma once
+
+#include "exec.hpp"
+
+namespace loom::hipvm
+{
+/// Operations of a START worth pooling.  Below, reading the pool costs about
+/// what START does (fib and Collatz: 3 operations, the cubic: 4).
+inline constexpr std::uint32_t kPoolMinOps = 24;
+
+template <typename K>
+struct StartPool
+{
+    static constexpr std::size_t none = ~std::size_t(0);
+
+    /// the instruction that sets register @p r to a literal for good in START
+    static constexpr std::size_t
+    literal(std::size_t r)
+    {
+        constexpr const auto& T  = ir::table_of<K>;
+        std::size_t           at = none;
+        for(std::size_t i = T.block[0].i0; i < std::size_t(T.block[0].i0 + T.block[0].ni); ++i)
+        {
+            const ir::Instr& in = T.instr[i];
+            if(in.kind != SK::compute || T.opnd[in.dst].slot != r) continue;
+            at = in.op == Op::mov && T.opnd[in.a0].lit ? i : none;
+        }
+        return at;
+    }
+
+    struct Map
+    {
+        std::array<std::uint16_t, 2 * ir::max_regs> reg{};  ///< register of each word
+        std::array<std::uint8_t, 2 * ir::max_regs>  half{}; ///< upper half of a 64-bit one
+        std::array<bool, ir::max_regs>              live{}; ///< live after START
+        std::size_t                                 n    = 0;
+        std::size_t                                 succ = 0; ///< successors but HALT
+        std::uint32_t                               next = 0; ///< the last of them
+        bool                                        back = false;
+    };
+
+    static constexpr Map map = []
+    {
+        constexpr const auto& T = ir::table_of<K>;
+        Map                   m;
+        ir::Bits              any{};
+        for(std::size_t j = 0; j < T.block[0].ns; ++j)
+        {
+            const auto s = T.succ[T.block[0].s0 + j];
+            if(s == ir::halt16) continue;
+            any = any | T.block[s].live_in;
+            if(m.succ == 0 || m.next != s) ++m.succ;
+            m.next = s;
+        }
+        for(std::size_t b = 0; b < T.nb; ++b)
+            for(std::size_t j = 0; j < T.block[b].ns; ++j)
+                m.back |= T.succ[T.block[b].s0 + j] == 0;
+        for(std::size_t r = 0; r < T.nr; ++r)
+        {
+            m.live[r] = any.test(r);
+            if(!m.live[r] || literal(r) != none) continue;
+            for(std::uint8_t h = 0; h < (T.reg[r].width == 8 ? 2 : 1); ++h)
+            {
+                m.reg[m.n]    = static_cast<std::uint16_t>(r);
+                m.half[m.n++] = h;
+            }
+        }
+        return m;
+    }();
+
+    static constexpr bool used =
+        ir::table_of<K>.block[0].ops >= kPoolMinOps && map.succ != 0 && !map.back;
+    /// columns: the words of the registers, the thread id, the next block
+    static constexpr std::size_t columns = used ? map.n + 1 + (map.succ > 1 ? 1 : 0) : 1;
+};
+
+template <typename K>
+__shared__ std::uint32_t start_pool[StartPool<K>::columns * 64];
+
+/// @brief Put this lane's thread, started, into row @p row of the pool.
+template <typename K>
+LOOM_DEVICE void
+pool_write(const Regs<K>& r, std::uint32_t pc, std::uint32_t tid, std::uint32_t row)
+{
+    using M = StartPool<K>;
+    [&]<std::size_t... W>(std::index_sequence<W...>)
+    {
+        ((start_pool<K>[W * 64 + row] = static_cast<std::uint32_t>(
+              r.template raw<M::map.reg[W]>() >> (M::map.half[W] ? 32 : 0))),
+         ...);
+    }(std::make_index_sequence<M::map.n>{});
+    start_pool<K>[M::map.n * 64 + row] = tid;
+    if constexpr(M::map.succ > 1) start_pool<K>[(M::map.n + 1) * 64 + row] = pc;
+}
+
+/// @brief Take the thread of row @p row into this lane; returns its id.
+template <typename K>
+LOOM_DEVICE std::uint32_t
+pool_read(Regs<K>& r, std::uint32_t& pc, std::uint32_t row)
+{
+    using M = StartPool<K>;
+    [&]<std::size_t... W>(std::index_sequence<W...>)
+    {
+        (
+            [&]
+            {
+                constexpr std::size_t R = M::map.reg[W];
+                const std::uint64_t   v = start_pool<K>[W * 64 + row];
+                if constexpr(M::map.half[W] != 0)
+                    r.template set_raw<R>((r.template raw<R>() & 0xFFFFFFFFull) | (v << 32));
+                else
+                    r.template set_raw<R>(v);
+            }(),
+            ...);
+    }(std::make_index_sequence<M::map.n>{});
+    std::uint32_t none = HALT, err = 0;
+    [&]<std::size_t... R>(std::index_sequence<R...>)
+    {
+        (
+            [&]
+            {
+                if constexpr(M::map.live[R] && M::literal(R) != M::none)
+                    exec_instr<K, M::literal(R)>(r, none, err);
+            }(),
+            ...);
+    }(std::make_index_sequence<ir::table_of<K>.nr>{});
+    if constexpr(M::map.succ > 1)
+        pc = start_pool<K>[(M::map.n + 1) * 64 + row];
+    else
+        pc = M::map.next;
+    return start_pool<K>[M::map.n * 64 + row];
+}
+} // namespace loom::hipvm

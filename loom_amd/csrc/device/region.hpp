@@ -15,13 +15,14 @@
 /// regions (11 vector instructions a trip); fib, 2^20 threads, 48 and 25 us.
 ///
 /// Leaders are START, the targets of back edges, and every block whose
-/// predecessors lie in different regions or in another loop.  A block joins
+/// predecessors lie in different regions or in another loop (or in a START
+/// that is pooled, pool.hpp).  A block joins
 /// the region of its predecessors only within the same set of loops: the
 /// code after a loop is a region of its own, which lanes leaving the loop at
 /// different trips reach together.
 #pragma once
 
-#include "exec.hpp"
+#include "pool.hpp"
 
 namespace loom::hipvm
 {
@@ -91,6 +92,8 @@ struct Regions
                             r = (r == NONE || r == m.of[p]) && in_loops[m.of[p]] == in_loops[b] ?
                                     m.of[p] :
                                     64u;
+            // a pooled START runs alone: its threads enter the sweep after it
+            if(r == 0 && StartPool<K>::used) r = 64u;
             m.of[b] = r < 64u ? static_cast<std::uint8_t>(r) : b;
             ++m.count[m.of[b]];
         }

@@ -27,6 +27,7 @@
 #pragma once
 
 #include "memregs.hpp"
+#include "pool.hpp"
 #include "region.hpp"
 
 #include <hip/hip_runtime.h>
@@ -852,10 +853,13 @@ sweep_region(Regs<K>& r, std::uint32_t& pc, std::uint32_t live_thr, PlainCtx& w)
 /// @brief POLICY_SWEEP runner: sweeps until every lane halted or, after a
 /// sweep, at most @p live_thr lanes are live (one sweep runs regardless when
 /// @p force is set).
-template <typename K, typename RF, typename Ctx>
+/// @p Pooled: no lane is ever at START (the pool ran it).
+template <typename K, bool Pooled, typename RF, typename Ctx>
 LOOM_DEVICE void
 run_sweep(RF& r, std::uint32_t& pc, std::uint32_t live_thr, bool force, Ctx& w)
 {
+    static_assert(!Pooled || !sweeps_regions<RF> || Regions<K>::map.count[0] == 1,
+                  "a lane could be at a block of START's region, which no sweep runs");
     if(!ballot(pc != HALT)) return;
     if(!force && live_thr && popc(ballot(pc != HALT)) <= live_thr) return;
     for(;;)
@@ -866,7 +870,9 @@ run_sweep(RF& r, std::uint32_t& pc, std::uint32_t live_thr, bool force, Ctx& w)
                 [&]
                 {
                     constexpr std::size_t B = ir::table_of<K>.order[R];
-                    if constexpr(sweeps_regions<RF>)
+                    if constexpr(Pooled && B == 0)
+                        return;
+                    else if constexpr(sweeps_regions<RF>)
                     {
                         if constexpr(Regions<K>::map.of[B] == B)
                             sweep_region<K, B>(r, pc, live_thr, w);
@@ -885,7 +891,7 @@ run_sweep(RF& r, std::uint32_t& pc, std::uint32_t live_thr, bool force, Ctx& w)
 
 /// @brief Run the wave under policy @p P (see run_to_threshold / run_topo /
 /// run_sweep).
-template <typename K, int P, typename RF, typename Ctx>
+template <typename K, int P, bool Pooled = false, typename RF, typename Ctx>
 LOOM_DEVICE void
 run_policy(RF& r, std::uint32_t& pc, std::uint32_t thr, std::uint32_t live_thr, bool force,
            Ctx& w)
@@ -893,7 +899,7 @@ run_policy(RF& r, std::uint32_t& pc, std::uint32_t thr, std::uint32_t live_thr, 
     if constexpr(P == POLICY_TOPO)
         run_topo<K>(r, pc, live_thr, force, w);
     else if constexpr(P == POLICY_SWEEP)
-        run_sweep<K>(r, pc, live_thr, force, w);
+        run_sweep<K, Pooled>(r, pc, live_thr, force, w);
     else
         run_to_threshold<K>(r, pc, thr, live_thr, force, w);
 }
@@ -1146,6 +1152,110 @@ fill_label(std::uint32_t label, Regs<K>& r, const char* q, std::uint64_t qcap,
 }
 
 // ---------------------------------------------------------------------------
+// refilling a wave's lanes
+// ---------------------------------------------------------------------------
+/// @brief Threads taken from an input: @p count of them, of which this lane
+/// of those that take some gets the k-th (at(k)).
+struct Taken
+{
+    std::uint32_t count = 0;
+    std::uint32_t head = 0, base = 0, more = 0; ///< head threads from base on, then from more on
+
+    LOOM_DEVICE std::uint32_t
+    at(std::uint32_t k) const
+    {
+        return k < head ? base + k : more + (k - head);
+    }
+};
+
+/// @brief The lanes of a wave that takes threads from an input (a callable
+/// want -> Taken) until it is exhausted: their threads, and the pool of
+/// started ones behind them where the kernel and the policy use one.
+template <typename K, int P, typename RF>
+struct Lanes
+{
+    static constexpr bool pooled = P == POLICY_SWEEP && StartPool<K>::used;
+
+    RF            r;
+    std::uint32_t pc   = HALT;
+    std::uint32_t tid  = 0;
+    bool          has  = false; ///< this lane holds a thread
+    bool          more = true;  ///< the input may hold more
+    std::uint32_t pool = 0;     ///< rows left in the pool
+    std::uint32_t row  = 0;     ///< the first of them
+
+    LOOM_DEVICE bool
+    input_left() const
+    {
+        return more || (pooled && pool != 0);
+    }
+
+    /// Start new threads in the lanes of @p empty; returns how many.
+    template <typename In, typename Ctx, typename Io>
+    LOOM_DEVICE std::uint32_t
+    refill(std::uint64_t empty, const Io& io, Ctx& w, In&& input, std::uint64_t& admitted)
+    {
+        const std::uint32_t want = popc(empty), k = rank_in(empty);
+        if constexpr(!pooled)
+        {
+            const Taken t = input(want);
+            if(!has && k < t.count)
+            {
+                tid = t.at(k);
+                load_inputs<K>(r, io.in, tid);
+                pc  = 0;
+                has = true;
+            }
+            admitted += t.count;
+            more = t.count != 0;
+            return t.count;
+        }
+        else
+        {
+            std::uint32_t given = 0;
+            while(given < want)
+            {
+                if(pool == 0)
+                {
+                    const Taken t = input(64u);
+                    more          = t.count != 0;
+                    if(!more) break;
+                    admitted += t.count;
+                    RF            s;
+                    std::uint32_t spc = HALT, stid = 0;
+                    const bool    mine = lane_id() < t.count;
+                    if(mine)
+                    {
+                        stid = t.at(lane_id());
+                        load_inputs<K>(s, io.in, stid);
+                        spc = 0;
+                    }
+                    run_block<K, 0>(s, spc, w);
+                    if(mine && spc == HALT) store_outputs<K>(s, io.out, stid);
+                    const std::uint64_t keep = ballot(spc != HALT);
+                    if(spc != HALT) pool_write<K>(s, spc, stid, rank_in(keep));
+                    // the rows are read by other lanes of this wave
+                    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+                    __builtin_amdgcn_wave_barrier();
+                    row  = 0;
+                    pool = popc(keep);
+                }
+                const std::uint32_t g = pool < want - given ? pool : want - given;
+                if(!has && k - given < g) // k >= given for the lanes still empty
+                {
+                    tid = pool_read<K>(r, pc, row + (k - given));
+                    has = true;
+                }
+                row += g;
+                pool -= g;
+                given += g;
+            }
+            return given;
+        }
+    }
+};
+
+// ---------------------------------------------------------------------------
 // hybrid form: pass kernel
 // ---------------------------------------------------------------------------
 /// @brief How a hybrid run's input is dealt to its waves, in batches of 64
@@ -1289,20 +1399,7 @@ next_batch(const HybridArgs& h, const Dealt& d, std::uint64_t n, Reservoir& res)
 }
 
 /// @brief Up to @p want threads from the reservoir (wave-uniform): the rest of
-/// the batch in hand and, if that is not enough, of the one after it.  The
-/// k-th of them is @p at(k).
-struct Taken
-{
-    std::uint32_t count = 0;
-    std::uint32_t head = 0, base = 0, more = 0; ///< head threads from base on, then from more on
-
-    LOOM_DEVICE std::uint32_t
-    at(std::uint32_t k) const
-    {
-        return k < head ? base + k : more + (k - head);
-    }
-};
-
+/// the batch in hand and, if that is not enough, of the one after it.
 LOOM_DEVICE Taken
 take_input(const HybridArgs& h, const Dealt& d, std::uint64_t n, Reservoir& res, std::uint32_t want)
 {
@@ -1367,52 +1464,39 @@ hybrid_pass_kernel(IoArgs io, CtlArgs c, HybridArgs h)
     std::uint64_t spill_rows = 0, spill_bytes = 0, fill_rows = 0, fill_bytes = 0,
                   admitted = 0, refills = 0, batches = 0, spill_failed = 0;
 
-    RegsOf<K, CNT> r;
-    std::uint32_t  pc  = HALT;
-    std::uint32_t  tid = 0;
-    bool           has = false;
-
     if constexpr(!RG)
     {
         // Without queues every wave takes input until none is left and then
         // finishes its lanes in place.  One call site of the claim and one of
         // the block code, which are inlined.
-        bool more = true;
+        Lanes<K, P, RegsOf<K, CNT>> l;
+        auto input = [&](std::uint32_t want) { return take_input(h, dealt, c.n, res, want); };
         for(;;)
         {
             if constexpr(CNT) flush_if_high(w);
-            const std::uint64_t live = ballot(has);
+            const std::uint64_t live = ballot(l.has);
             bool                took = false;
-            if(more && ~live && (c.refill || !live))
+            if(l.input_left() && ~live && (c.refill || !live))
             {
-                const Taken t = take_input(h, dealt, c.n, res, popc(~live));
-                took          = t.count != 0;
-                more          = took;
-                if(took)
-                {
-                    const std::uint32_t k = rank_in(~live);
-                    if(!has && k < t.count)
-                    {
-                        tid = t.at(k);
-                        load_inputs<K>(r, io.in, tid);
-                        pc  = 0;
-                        has = true;
-                    }
-                    admitted += t.count;
-                    ++(live ? refills : batches);
-                }
+                took = l.refill(~live, io, w, input, admitted) != 0;
+                if(took) ++(live ? refills : batches);
             }
-            if(!ballot(has)) break;
-            run_policy<K, P>(r, pc, took ? c.thr : 0u, took ? c.live_thr : 0u, true, w);
+            if(!ballot(l.has)) break;
+            run_policy<K, P, l.pooled>(l.r, l.pc, took ? c.thr : 0u, took ? c.live_thr : 0u, true, w);
             if(w.over) break;
-            if(has && pc == HALT)
+            if(l.has && l.pc == HALT)
             {
-                store_outputs<K>(r, io.out, tid);
-                has = false;
+                store_outputs<K>(l.r, io.out, l.tid);
+                l.has = false;
             }
         }
     }
     else
+    {
+        Regs<K>       r;
+        std::uint32_t pc  = HALT;
+        std::uint32_t tid = 0;
+        bool          has = false;
         for(;;)
         {
             if constexpr(CNT) flush_if_high(w);
@@ -1528,6 +1612,7 @@ hybrid_pass_kernel(IoArgs io, CtlArgs c, HybridArgs h)
             }
             if(w.over) break;
         }
+    }
     flush_stats(w);
     if(CNT && c.stats && lane == 0)
     {

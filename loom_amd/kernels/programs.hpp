@@ -143,6 +143,52 @@ TKERNEL2(nested, a, b)
     IPJMP2(f, HALT, outer)
 TKERNEL_END2(s, c);
 
+// A long START that goes four ways (one of them out), with registers it sets
+// to literals, sets twice and leaves to later blocks.
+template <std::unsigned_integral T>
+TKERNEL2(started, a, b)
+    IMOV(n, 3),
+    IMOV(s, 7),
+    IMOV(c, 0),
+    IMOV(d, 1),
+    ILSHFT(t, a, 13),
+    IXOR(x, a, t),
+    IRSHFT(t, x, 7),
+    IXOR(x, x, t),
+    ILSHFT(t, x, 17),
+    IXOR(x, x, t),
+    IMUL(y, b, 0x9E3779B9),
+    IADD(y, y, x),
+    IRSHFT(t, y, 11),
+    IXOR(y, y, t),
+    IMUL(y, y, 0x85EBCA6B),
+    IRSHFT(t, y, 13),
+    IXOR(y, y, t),
+    ILSHFT(t, y, 3),
+    IADD(y, y, t),
+    IXOR(x, x, y),
+    IRSHFT(t, x, 5),
+    IADD(x, x, t),
+    IADD(s, s, x),
+    IMOV(d, 9),
+    IBAND(k, y, 3),
+    IPJMP4(k, spin, once, HALT, twice),
+    LABEL(twice),
+    IADD(n, n, 4),
+    LABEL(spin),
+    IMUL(s, s, 5),
+    IADD(s, s, d),
+    IADD(c, c, 1),
+    ISUB(n, n, 1),
+    IBAND(f, s, 64),
+    ICMOV(n, f, 0, n),
+    INEQ(f, n, 0),
+    IPJMP2(f, once, spin),
+    LABEL(once),
+    IXOR(s, s, x),
+    IADD(c, c, 100)
+TKERNEL_END3(s, c, d);
+
 // Integer op mix, straight-line: every binary integer operation of the
 // contract on (a, b), folded into several outputs.
 template <std::unsigned_integral T>

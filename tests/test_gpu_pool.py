@@ -1,0 +1,55 @@
+"""Refilling from a wave's pool of started threads (kernels with a long START,
+sweep policy): outputs equal the oracle's bit for bit and every thread's work
+is counted once, for inputs below a wave, a few rows past a pool, and many
+pools per wave; refilled at any threshold, at the last lane and not at all; a
+START that halts for some threads and goes several ways for others."""
+import numpy as np
+import pytest
+
+import loom_amd
+from loom_amd import abi, workloads
+from tests import oracle_lib as O
+
+pytestmark = pytest.mark.gpu
+
+
+def started(n):
+    rng = np.random.default_rng(n)
+    return [rng.integers(0, 1 << 64, n, dtype=np.uint64) for _ in range(2)]
+
+
+def frame(n):
+    sid = np.arange(n, dtype=np.uint32) * np.uint32(7)
+    return [sid, np.full(n, workloads.pt_job(61, 43, 255), np.uint32)]
+
+
+INPUTS = {"started_u64": started, "smallpt9_f32": frame}
+FORMS = [dict(live_threshold=48), dict(live_threshold=63), dict(live_threshold=0),
+         dict(live_threshold=60, waves_per_cu=1), dict(refill=False),
+         dict(live_threshold=32, reconv=abi.RECONV_TOPO)]
+WORK = (abi.C_ACTIVE_OPS, abi.C_THREAD_STEPS, abi.C_ACTIVE_FLOPS)
+
+
+def bits(a):
+    return a.view(np.uint32) if a.dtype == np.float32 else a
+
+
+@pytest.mark.parametrize("name", list(INPUTS))
+def test_pool_matches_oracle(gpu, name):
+    for n in (1, 63, 64, 65, 127, 129, 4 * 256 * 64 + 17):
+        ins = INPUTS[name](n)
+        want, err = O.run(name, ins)
+        assert err == 0
+        base = loom_amd.run(name, abi.MODE_COMPACT, ins,
+                            params=loom_amd.make_params(reconv=abi.RECONV_SWEEP))
+        for params in FORMS:
+            for stats in (True, False):
+                print(f"[gpu] pool {name} n={n} {params} stats {stats}", flush=True)
+                r = loom_amd.run(name, abi.MODE_HYBRID, ins, params=loom_amd.make_params(
+                    mode=abi.MODE_HYBRID, stats=stats, **params))
+                for g, w in zip(r.outputs, want):
+                    assert np.array_equal(bits(g), bits(w)), (name, n, params)
+                if stats:
+                    assert r.counters[abi.C_ADMITTED] == n
+                    for c in WORK:
+                        assert r.counters[c] == base.counters[c], (name, n, params, c)
