@@ -315,8 +315,9 @@ int loom_ctx_synchronize(loom_context* ctx);
  *               empties the rest;
  *   step        one launch: every live slot runs under loom_params.reconv
  *               until at most live_threshold lanes of its wave are live
- *               (0: to HALT) or max_steps dispatches were made; threads keep
- *               their registers between steps;
+ *               (0: to HALT; in a wave that had no more to begin with, until
+ *               half of those halted) or max_steps dispatches were made;
+ *               threads keep their registers between steps;
  *   sort        reports whether an exchange is available: at least 64 slots
  *               halted since the last exchange, or some halted and none live;
  *   exchange    for m = min(n, halted) finished threads, in the order they

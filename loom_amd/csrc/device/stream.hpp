@@ -117,11 +117,19 @@ store_state(const Regs<K>& r, const StreamArgs& a, std::uint64_t slot)
     }(std::make_index_sequence<ir::table_of<K>.nr>{});
 }
 
+/// Dispatches after which a step ends for a wave of few live slots, so that
+/// the host sees the stream again also where none of them halts soon.
+inline constexpr std::uint64_t kFewSteps = 1u << 16;
+
 /// @brief One step of the stream: each wave owns 64 consecutive slots, loads
 /// the registers of its live slots, runs them under policy @p P until at
 /// most `live_thr` of them are live (or the dispatch budget of the step is
 /// spent: a step budget only ends the step, the threads keep their state),
 /// writes the registers back and appends the slots that halted to the ring.
+/// A wave that has no more live slots than that to begin with runs until half
+/// of them have halted: ending after a sweep, as it would otherwise, hands
+/// the host nothing to exchange and costs it a step all the same (Collatz,
+/// 300,007 threads through 65,536 slots: 4.35 ms a stream, and 2.06 so).
 template <typename K, int P, bool CNT = true>
 __global__ __launch_bounds__(64) void
 stream_step_kernel(StreamArgs a, CtlArgs c)
@@ -138,8 +146,11 @@ stream_step_kernel(StreamArgs a, CtlArgs c)
         load_state<K>(r, a, slot);
         pc = pc0;
     }
+    const std::uint32_t lanes = popc(ballot(live));
+    const bool          few   = lanes <= c.live_thr;
+    if(few && c.max_steps > kFewSteps) c.max_steps = kFewSteps;
     CtxOf<CNT> w(c);
-    run_policy<K, P>(r, pc, c.thr, c.live_thr, true, w);
+    run_policy<K, P>(r, pc, c.thr, few ? lanes / 2u : c.live_thr, true, w);
     if(live)
     {
         store_state<K>(r, a, slot);
