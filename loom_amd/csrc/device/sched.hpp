@@ -940,6 +940,85 @@ compact_kernel(IoArgs io, CtlArgs c)
     raise_errors(w.err, w.over, c);
 }
 
+/// @brief Straight-line kernels: threads per lane of compact_wide_kernel.
+inline constexpr int kWide = 4;
+
+/// @brief kWide consecutive elements of a column, as vectors of 16 bytes.
+template <typename V>
+struct alignas(sizeof(V) * kWide < 16 ? sizeof(V) * kWide : 16) WideCells
+{
+    V v[kWide];
+};
+
+/// @brief The compact form of a straight-line kernel whose columns are its
+/// cost: a lane takes kWide consecutive threads, so that a column of 4-byte
+/// elements is read and written 16 bytes at a time and the loads of all its
+/// threads are in flight at once.  For runs that count no work, over columns
+/// aligned to WideCells (launch_compact).
+template <typename K>
+__global__ __launch_bounds__(256) void
+compact_wide_kernel(IoArgs io, CtlArgs c)
+{
+    sct_table_init<K>();
+    const std::uint64_t first = (std::uint64_t(blockIdx.x) * blockDim.x + threadIdx.x) * kWide;
+    PlainCtx            w(c);
+    Regs<K>             r[kWide];
+    const bool          whole = first + kWide <= c.n;
+    if(whole)
+    {
+        [&]<std::size_t... J>(std::index_sequence<J...>)
+        {
+            (
+                [&]
+                {
+                    using V        = ctype<ir::table_of<K>.in_ty[J]>;
+                    const auto cell = *reinterpret_cast<const WideCells<V>*>(
+                        static_cast<const V*>(io.in[J]) + first);
+#pragma unroll
+                    for(int t = 0; t < kWide; ++t)
+                        r[t].template set<ir::table_of<K>.in_slot[J], V>(cell.v[t]);
+                }(),
+                ...);
+        }(std::make_index_sequence<ir::table_of<K>.nin>{});
+    }
+    else
+    {
+#pragma unroll
+        for(int t = 0; t < kWide; ++t)
+            if(first + t < c.n) load_inputs<K>(r[t], io.in, first + t);
+    }
+#pragma unroll
+    for(int t = 0; t < kWide; ++t)
+    {
+        std::uint32_t pc = 0;
+        if(first + t < c.n) exec_block<K, 0>(r[t], pc, w.err);
+    }
+    if(whole)
+    {
+        [&]<std::size_t... J>(std::index_sequence<J...>)
+        {
+            (
+                [&]
+                {
+                    using V = ctype<ir::table_of<K>.out_ty[J]>;
+                    WideCells<V> cell;
+#pragma unroll
+                    for(int t = 0; t < kWide; ++t)
+                        cell.v[t] = r[t].template get<ir::table_of<K>.out_slot[J], V>();
+                    *reinterpret_cast<WideCells<V>*>(static_cast<V*>(io.out[J]) + first) = cell;
+                }(),
+                ...);
+        }(std::make_index_sequence<ir::table_of<K>.nout>{});
+    }
+    else
+    {
+#pragma unroll
+        for(int t = 0; t < kWide; ++t)
+            if(first + t < c.n) store_outputs<K>(r[t], io.out, first + t);
+    }
+    raise_errors(w.err, false, c);
+}
+
 /// @brief The register file of a compact run in device memory: column r of
 /// `rows` cells at base + rows * CellLayout<K>::off[r].
 struct MemArgs

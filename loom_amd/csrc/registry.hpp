@@ -124,11 +124,62 @@ make_batch(const char* name)
     return e;
 }
 
+/// @brief Kernel @p K is straight-line over columns of at most 4 bytes, and
+/// reads no register that is not an input (load_inputs would have to clear
+/// it).  Wider elements fill the memory pipeline one per lane, and four
+/// threads' registers, above all those of integer divisions (some forty
+/// instructions each), cost occupancy: 2^24 threads, microseconds one per lane
+/// and kWide per lane, threefry2x32 94.7 and 78.3 (402 MB: the rate of a large
+/// copy), fp_mix f32 130 and 115, sincos f32 42 and 32, sct_range f32 81 and
+/// 65, literal_div f32 102 and 96; but int_mix u32 101 and 116, u64 210 and 234.
+template <typename K>
+inline constexpr bool wide_kernel = []
+{
+    constexpr const auto& T = ir::table_of<K>;
+    if(!T.straightline || T.nb != 1) return false;
+    for(std::size_t r = 0; r < T.nr; ++r)
+        if(T.block[0].live_in.test(r) && !T.reg[r].input) return false;
+    for(std::size_t k = 0; k < T.nin; ++k)
+        if(ir::ty_size(T.in_ty[k]) > 4) return false;
+    for(std::size_t k = 0; k < T.nout; ++k)
+        if(ir::ty_size(T.out_ty[k]) > 4) return false;
+    for(std::size_t i = 0; i < T.ni; ++i)
+        if((T.instr[i].op == ir::Op::div || T.instr[i].op == ir::Op::mod) &&
+           !ir::ty_float(T.instr[i].ety))
+            return false;
+    return true;
+}();
+
+/// Threads from which a straight-line kernel runs kWide per lane: two rounds
+/// of the chip's lanes (256 CUs x 2048) after the division (threefry2x32,
+/// 2^22 threads: 23.6 and 22.0 us).
+inline constexpr std::uint64_t kWideThreads = std::uint64_t(kWide) << 20;
+
+/// @brief Every column of @p io is aligned for kWide elements at once.
+template <typename K>
+bool
+wide_columns(const IoArgs& io)
+{
+    constexpr const auto& T  = ir::table_of<K>;
+    auto                  ok = [](const void* p, ir::Ty t)
+    {
+        const std::size_t b = ir::ty_size(t) * kWide;
+        return reinterpret_cast<std::uintptr_t>(p) % (b < 16 ? b : 16) == 0;
+    };
+    bool all = true;
+    for(std::size_t k = 0; k < T.nin; ++k) all = all && ok(io.in[k], T.in_ty[k]);
+    for(std::size_t k = 0; k < T.nout; ++k) all = all && ok(io.out[k], T.out_ty[k]);
+    return all;
+}
+
 template <typename K, int P>
 hipError_t
 launch_compact(const IoArgs& io, const CtlArgs& c, hipStream_t s)
 {
     if(c.n == 0) return hipSuccess;
+    if constexpr(wide_kernel<K>)
+        if(plain_run(c) && c.n >= kWideThreads && wide_columns<K>(io))
+            return launch(compact_wide_kernel<K>, (c.n + 256 * kWide - 1) / (256 * kWide), 256, s, io, c);
     const std::uint64_t blocks = (c.n + 255) / 256;
     // a run that counts no work takes the kernel that sweeps regions where
     // the kernel has small blocks (the same kernel otherwise)
