@@ -21,6 +21,19 @@ namespace loom::hipvm
 {
 inline constexpr std::uint32_t kMaxJobs = 64;
 
+/// @brief Waves per SIMD that a batch kernel with member @p K is compiled to
+/// allow at least (as waves_hint; LOOM_HIP_BATCH_WAVES_HINT): the largest of
+/// its members' hints.
+template <typename K>
+inline constexpr int batch_waves_hint = 1;
+template <typename... Ks>
+inline constexpr int batch_waves = []
+{
+    int w = 1;
+    ((w = batch_waves_hint<Ks> > w ? batch_waves_hint<Ks> : w), ...);
+    return w;
+}();
+
 /// @brief One job of a batch (device copy of loom_job).
 struct JobDesc
 {
@@ -125,7 +138,7 @@ struct BatchSet
 /// @brief The persistent batch kernel over the kernels @p Ks (policy @p P;
 /// CNT: with work counts, else for runs that count none, see plain_run).
 template <int P, bool CNT, typename... Ks>
-__global__ __launch_bounds__(64) void
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(batch_waves<Ks...>))) void
 batch_kernel(CtlArgs c, BatchArgs a)
 {
     (sct_table_init<Ks>(), ...);

@@ -5,10 +5,10 @@
 
 #include "../kernels/catalog.hpp"
 
-// The path tracer's pass kernel needs 132 VGPRs left to itself (three waves
-// per SIMD).  Held to 128 (four waves, two values spilled) it renders the
-// 1024x768x64 frame in 8.30 ms instead of 9.05; held to 96 (five waves, 32
-// bytes spilled) in 8.11 ms; held to 80 (six waves, 76 bytes) in 8.24 ms.
+// The path tracer's pass kernel left to itself runs three waves per SIMD.
+// The 1024x768x64 frame takes 6.90 ms held to 128 VGPRs (four waves), 6.44
+// held to 96 (five) and 6.42 held to 80 (six): the same within what two boxes
+// differ by, so the one with fewer spills stays.
 LOOM_HIP_WAVES_HINT(5, loom_amd::smallpt::smallpt9<float>);
 // With the regroup paths it needs 133: held to 128 (four waves) a
 // regrouping frame with refill takes 8.5 ms, held to 96 (five waves, 40

@@ -423,6 +423,12 @@ make_entry(const char* name)
     template <>                                                                        \
     inline constexpr int ::loom::hipvm::regroup_waves_hint<__VA_ARGS__> = (W)
 
+/// @brief The same for the batch kernels that kernel type `...` is a member of
+/// (before their LOOM_HIP_REGISTER_BATCH).
+#define LOOM_HIP_BATCH_WAVES_HINT(W, ...)                                             \
+    template <>                                                                        \
+    inline constexpr int ::loom::hipvm::batch_waves_hint<__VA_ARGS__> = (W)
+
 /// @brief Lower kernel type `...` and register it under @p NAME.
 #define LOOM_HIP_REGISTER(NAME, ...) LOOM_HIP_REGISTER_I(__COUNTER__, NAME, __VA_ARGS__)
 
