@@ -9,9 +9,8 @@ namespace P = loom_amd::programs;
 namespace S = loom_amd::smallpt;
 
 // The path tracer's batch kernel fits five waves per SIMD by itself; held to
-// six, 16 jobs of frames, fib and Collatz take 2.25 ms instead of 2.30: its
-// Collatz and fib waves gain more from the sixth wave than the path tracer's
-// lose to the spills.
+// six, 16 jobs of frames, fib and Collatz take 2.21 ms instead of 2.29 (a pass
+// kernel of the path tracer alone is the same at both).
 LOOM_HIP_BATCH_WAVES_HINT(6, S::smallpt9<float>);
 
 // the mixed benchmark batch: path-trace frames with fib and Collatz jobs
