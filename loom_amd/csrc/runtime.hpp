@@ -98,7 +98,7 @@ struct loom_context
     hipEvent_t     ev[4]{};
     std::vector<hipEvent_t> pass_ev;
     loom::hipvm::JobDesc*  jobs = nullptr; ///< device job table of direct batch runs
-    loom::hipvm::JobDesc*  host_jobs = nullptr; ///< pinned: the table as the host wrote it
+    loom::hipvm::JobDesc*  host_jobs = nullptr; ///< the table as the host wrote it, in the block of err
     loom::hipvm::BatchCtl* bctl = nullptr;
     /// background copies: tickets of outstanding copies, oldest first
     std::deque<std::pair<std::uint64_t, hipEvent_t>> tickets;
