@@ -1269,7 +1269,8 @@ struct Lanes
         return more || (pooled && pool != 0);
     }
 
-    /// Start new threads in the lanes of @p empty; returns how many.
+    /// Start new threads in the lanes of @p empty; returns how many.  The
+    /// wave's dispatch budget may end in it (w.over), with threads taken.
     template <typename In, typename Ctx, typename Io>
     LOOM_DEVICE std::uint32_t
     refill(std::uint64_t empty, const Io& io, Ctx& w, In&& input, std::uint64_t& admitted)
@@ -1311,6 +1312,15 @@ struct Lanes
                     }
                     run_block<K, 0>(s, spc, w);
                     if(mine && spc == HALT) store_outputs<K>(s, io.out, stid);
+                    // where START halts most threads this loop runs many of
+                    // them: the budget and the counters' bounds hold here too
+                    // (a run that counts no work has neither: its budget is
+                    // 2^40 dispatches, its batches are at most 2^26)
+                    if constexpr(!std::is_same_v<Ctx, PlainCtx>)
+                    {
+                        segment_check(w);
+                        if(w.over) break;
+                    }
                     const std::uint64_t keep = ballot(spc != HALT);
                     if(spc != HALT) pool_write<K>(s, spc, stid, rank_in(keep));
                     // the rows are read by other lanes of this wave
@@ -1558,6 +1568,7 @@ hybrid_pass_kernel(IoArgs io, CtlArgs c, HybridArgs h)
             if(l.input_left() && ~live && (c.refill || !live))
             {
                 took = l.refill(~live, io, w, input, admitted) != 0;
+                if(CNT && w.over) break;
                 if(took) ++(live ? refills : batches);
             }
             if(!ballot(l.has)) break;

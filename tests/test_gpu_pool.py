@@ -53,3 +53,29 @@ def test_pool_matches_oracle(gpu, name):
                     assert r.counters[abi.C_ADMITTED] == n
                     for c in WORK:
                         assert r.counters[c] == base.counters[c], (name, n, params, c)
+
+
+def test_budget_holds_where_start_halts(gpu):
+    """Every thread halts in START, so a wave refills until its input is gone
+    and no other block runs: 40 STARTs a wave are over a budget of 8, and under
+    one of 1000 they give the outputs and the counts of the compact form."""
+    draw = started(1 << 15)
+    want, _ = O.run("started_u64", draw)
+    halts = np.flatnonzero(want[1] == 0)  # no other block ran
+    rows = np.resize(halts, 40 * 256 * 64)
+    ins, want = [a[rows] for a in draw], [w[rows] for w in want]
+
+    def run(mode, **p):
+        print(f"[gpu] all threads halt in START: mode {mode} {p}", flush=True)
+        return loom_amd.run("started_u64", mode, ins, params=loom_amd.make_params(
+            mode=mode, reconv=abi.RECONV_SWEEP, waves_per_cu=1, **p))
+
+    with pytest.raises(abi.LoomError, match="0x2"):
+        run(abi.MODE_HYBRID, max_steps=8)
+    base = run(abi.MODE_COMPACT)
+    for p in (dict(max_steps=1000), dict(), dict(stats=False), dict(refill=False)):
+        r = run(abi.MODE_HYBRID, **p)
+        for g, w in zip(r.outputs, want):
+            assert np.array_equal(g, w), p
+        for c in WORK:
+            assert r.counters[c] == (base.counters[c] if p.get("stats", True) else 0), (p, c)
