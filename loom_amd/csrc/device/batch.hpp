@@ -117,7 +117,7 @@ run_job(const BatchArgs& a, std::uint32_t j, const CtlArgs& c, CtxOf<CNT>& w, st
         if constexpr(CNT) flush_if_high(w);
         const std::uint64_t live = ballot(l.has);
         if(~live && l.input_left() && l.refill(~live, J[j], w, input, admitted)) force = true;
-        if((CNT && w.over) || !ballot(l.has)) return;
+        if((l.pooled && CNT && w.over) || !ballot(l.has)) return;
         run_policy<K, P, l.pooled>(l.r, l.pc, 0, l.input_left() ? c.live_thr : 0u, force, w);
         force = false;
         if(l.has && l.pc == HALT)

@@ -1568,7 +1568,7 @@ hybrid_pass_kernel(IoArgs io, CtlArgs c, HybridArgs h)
             if(l.input_left() && ~live && (c.refill || !live))
             {
                 took = l.refill(~live, io, w, input, admitted) != 0;
-                if(CNT && w.over) break;
+                if(l.pooled && CNT && w.over) break;
                 if(took) ++(live ? refills : batches);
             }
             if(!ballot(l.has)) break;
