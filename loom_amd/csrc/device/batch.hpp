@@ -21,16 +21,20 @@ namespace loom::hipvm
 {
 inline constexpr std::uint32_t kMaxJobs = 64;
 
-/// @brief Waves per SIMD that a batch kernel with member @p K is compiled to
-/// allow at least (as waves_hint; LOOM_HIP_BATCH_WAVES_HINT): the largest of
-/// its members' hints.
+/// @brief Waves per SIMD that the sweep policy's batch kernels with member
+/// @p K are compiled to allow at least (as waves_hint;
+/// LOOM_HIP_BATCH_WAVES_HINT): the largest of their members' hints.  The
+/// other policies keep more registers live across a dispatch and are left to
+/// the compiler: held to the path tracer's hint they spill 40 to 52 bytes a
+/// lane (16 mixed jobs of 20,011 threads, left alone and held: 698 and 828 us
+/// under the topological policy, 888 and 1064 under successor-major).
 template <typename K>
 inline constexpr int batch_waves_hint = 1;
-template <typename... Ks>
+template <int P, typename... Ks>
 inline constexpr int batch_waves = []
 {
     int w = 1;
-    ((w = batch_waves_hint<Ks> > w ? batch_waves_hint<Ks> : w), ...);
+    if constexpr(P == POLICY_SWEEP) ((w = batch_waves_hint<Ks> > w ? batch_waves_hint<Ks> : w), ...);
     return w;
 }();
 
@@ -138,7 +142,7 @@ struct BatchSet
 /// @brief The persistent batch kernel over the kernels @p Ks (policy @p P;
 /// CNT: with work counts, else for runs that count none, see plain_run).
 template <int P, bool CNT, typename... Ks>
-__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(batch_waves<Ks...>))) void
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(batch_waves<P, Ks...>))) void
 batch_kernel(CtlArgs c, BatchArgs a)
 {
     (sct_table_init<Ks>(), ...);

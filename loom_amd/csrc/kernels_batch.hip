@@ -8,8 +8,8 @@
 namespace P = loom_amd::programs;
 namespace S = loom_amd::smallpt;
 
-// The path tracer's batch kernel fits five waves per SIMD by itself; held to
-// six, 16 jobs of frames, fib and Collatz take 2.21 ms instead of 2.29 (a pass
+// The path tracer's sweeping batch kernel fits five waves per SIMD by itself;
+// held to six, 16 jobs of frames, fib and Collatz take 2.21 ms instead of 2.29 (a pass
 // kernel of the path tracer alone is the same at both).
 LOOM_HIP_BATCH_WAVES_HINT(6, S::smallpt9<float>);
 

@@ -423,8 +423,8 @@ make_entry(const char* name)
     template <>                                                                        \
     inline constexpr int ::loom::hipvm::regroup_waves_hint<__VA_ARGS__> = (W)
 
-/// @brief The same for the batch kernels that kernel type `...` is a member of
-/// (before their LOOM_HIP_REGISTER_BATCH).
+/// @brief The same for the sweep policy's batch kernels that kernel type `...`
+/// is a member of (before their LOOM_HIP_REGISTER_BATCH).
 #define LOOM_HIP_BATCH_WAVES_HINT(W, ...)                                             \
     template <>                                                                        \
     inline constexpr int ::loom::hipvm::batch_waves_hint<__VA_ARGS__> = (W)
