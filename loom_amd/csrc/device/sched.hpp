@@ -414,10 +414,10 @@ run_block(RF& r, std::uint32_t& pc, Ctx& w)
 {
     constexpr ir::Block blk = ir::table_of<K>.block[B];
     static_assert(blk.flops <= 2u * blk.ops, "flops exceed twice the op count");
-    w.disp += 1;
     if constexpr(std::is_same_v<Ctx, PlainCtx>)
     {
         if(pc == B) exec_on<K, B>(r, pc, w.err);
+        w.disp += 1;
         return;
     }
     else if constexpr(blk.ops >= kScalarStepOps)
@@ -436,6 +436,7 @@ run_block(RF& r, std::uint32_t& pc, Ctx& w)
         if constexpr(blk.flops != 0) w.lane_flops += blk.flops;
     }
     w.slots += 64u * blk.ops;
+    w.disp += 1;
 }
 
 /// @brief True when HALT is a successor of block @p B.
