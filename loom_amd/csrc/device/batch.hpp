@@ -83,8 +83,9 @@ claim_job_chunk(BatchCtl* ctl, const JobDesc* J, std::uint32_t j, std::uint32_t 
 }
 
 /// @brief Run job @p j (kernel K) on this wave until the job has no more
-/// threads to admit and every lane halted.
-template <typename K, int P, bool CNT>
+/// threads to admit and every lane halted: its pool of started threads is
+/// empty again then, so all jobs share one.
+template <typename K, int P, bool CNT, std::size_t Columns>
 LOOM_DEVICE void
 run_job(const BatchArgs& a, std::uint32_t j, const CtlArgs& c, CtxOf<CNT>& w, std::uint64_t& admitted)
 {
@@ -98,8 +99,8 @@ run_job(const BatchArgs& a, std::uint32_t j, const CtlArgs& c, CtxOf<CNT>& w, st
     std::uint32_t rcount = 0;
     bool          exhausted = false;
 
-    Lanes<K, P, RegsOf<K, CNT>> l;
-    bool                        force = true;
+    Lanes<K, P, RegsOf<K, CNT>, Columns> l;
+    bool                                 force = true;
 
     auto input = [&](std::uint32_t want)
     {
@@ -163,7 +164,7 @@ batch_kernel(CtlArgs c, BatchArgs a)
         (
             [&]
             {
-                if(m == idx) run_job<Ks, P, CNT>(a, j, c, w, admitted);
+                if(m == idx) run_job<Ks, P, CNT, pool_columns<Ks...>>(a, j, c, w, admitted);
                 ++idx;
             }(),
             ...);

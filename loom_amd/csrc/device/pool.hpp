@@ -15,7 +15,8 @@
 /// lanes, 72% of the lanes active), 6.44 with it (refilled at 60, 81%).
 ///
 /// Used where it pays: START of at least kPoolMinOps operations that no other
-/// block jumps back to, in waves that own their workgroup's LDS.
+/// block jumps back to, with few enough words live after it (lds_per_wave), in
+/// waves that own their workgroup's LDS.
 #pragma once
 
 #include "exec.hpp"
@@ -25,6 +26,36 @@ namespace loom::hipvm
 /// Operations of a START worth pooling.  Below, reading the pool costs about
 /// what START does (fib and Collatz: 3 operations, the cubic: 4).
 inline constexpr std::uint32_t kPoolMinOps = 24;
+
+/// @brief 32-bit words of the registers in @p live.
+template <typename K>
+constexpr std::size_t
+words_of(const ir::Bits& live)
+{
+    std::size_t n = 0;
+    for(std::size_t r = 0; r < ir::table_of<K>.nr; ++r)
+        if(live.test(r)) n += ir::table_of<K>.reg[r].width == 8 ? 2 : 1;
+    return n;
+}
+
+/// @brief LDS that a one-wave workgroup of @p K may use before it holds fewer
+/// waves than registers allow.  What is live at a block is in VGPRs there, 512
+/// a lane for all waves of a SIMD, of which eight fit at most; a CU has four
+/// SIMDs and 160 KB of LDS in granules of 1280 bytes: 5120 bytes (20 words a
+/// lane) where all eight fit, more for kernels with much live state.
+template <typename K>
+inline constexpr std::size_t lds_per_wave = []
+{
+    std::size_t words = 1;
+    for(std::size_t b = 0; b < ir::table_of<K>.nb; ++b)
+    {
+        const std::size_t w = words_of<K>(ir::table_of<K>.block[b].live_in);
+        words               = w > words ? w : words;
+    }
+    const std::size_t fit   = 512 / ((words + 7) / 8 * 8);
+    const std::size_t waves = fit < 1 ? 1 : (fit > 8 ? 8 : fit);
+    return 160 * 1024 / (4 * waves) / 1280 * 1280;
+}();
 
 template <typename K>
 struct StartPool
@@ -86,33 +117,45 @@ struct StartPool
         return m;
     }();
 
-    static constexpr bool used =
-        ir::table_of<K>.block[0].ops >= kPoolMinOps && map.succ != 0 && !map.back;
     /// columns: the words of the registers, the thread id, the next block
-    static constexpr std::size_t columns = used ? map.n + 1 + (map.succ > 1 ? 1 : 0) : 1;
+    static constexpr std::size_t columns = map.n + 1 + (map.succ > 1 ? 1 : 0);
+
+    static constexpr bool used =
+        ir::table_of<K>.block[0].ops >= kPoolMinOps && map.succ != 0 && !map.back &&
+        columns * 256 + SctTable<K>::words * 4 <= lds_per_wave<K>;
 };
 
-template <typename K>
-__shared__ std::uint32_t start_pool[StartPool<K>::columns * 64];
+/// @brief Columns of the pool of a wave that runs the kernels @p Ks one after
+/// the other: the largest of theirs.
+template <typename... Ks>
+inline constexpr std::size_t pool_columns = []
+{
+    std::size_t n = 1;
+    ((n = StartPool<Ks>::used && StartPool<Ks>::columns > n ? StartPool<Ks>::columns : n), ...);
+    return n;
+}();
 
-/// @brief Put this lane's thread, started, into row @p row of the pool.
-template <typename K>
+template <std::size_t Columns>
+__shared__ std::uint32_t start_pool[Columns * 64];
+
+/// @brief Put this lane's thread, started, into row @p row of the pool @p C.
+template <typename K, std::size_t C>
 LOOM_DEVICE void
 pool_write(const Regs<K>& r, std::uint32_t pc, std::uint32_t tid, std::uint32_t row)
 {
     using M = StartPool<K>;
     [&]<std::size_t... W>(std::index_sequence<W...>)
     {
-        ((start_pool<K>[W * 64 + row] = static_cast<std::uint32_t>(
+        ((start_pool<C>[W * 64 + row] = static_cast<std::uint32_t>(
               r.template raw<M::map.reg[W]>() >> (M::map.half[W] ? 32 : 0))),
          ...);
     }(std::make_index_sequence<M::map.n>{});
-    start_pool<K>[M::map.n * 64 + row] = tid;
-    if constexpr(M::map.succ > 1) start_pool<K>[(M::map.n + 1) * 64 + row] = pc;
+    start_pool<C>[M::map.n * 64 + row] = tid;
+    if constexpr(M::map.succ > 1) start_pool<C>[(M::map.n + 1) * 64 + row] = pc;
 }
 
 /// @brief Take the thread of row @p row into this lane; returns its id.
-template <typename K>
+template <typename K, std::size_t C>
 LOOM_DEVICE std::uint32_t
 pool_read(Regs<K>& r, std::uint32_t& pc, std::uint32_t row)
 {
@@ -123,7 +166,7 @@ pool_read(Regs<K>& r, std::uint32_t& pc, std::uint32_t row)
             [&]
             {
                 constexpr std::size_t R = M::map.reg[W];
-                const std::uint64_t   v = start_pool<K>[W * 64 + row];
+                const std::uint64_t   v = start_pool<C>[W * 64 + row];
                 if constexpr(M::map.half[W] != 0)
                     r.template set_raw<R>((r.template raw<R>() & 0xFFFFFFFFull) | (v << 32));
                 else
@@ -143,9 +186,9 @@ pool_read(Regs<K>& r, std::uint32_t& pc, std::uint32_t row)
             ...);
     }(std::make_index_sequence<ir::table_of<K>.nr>{});
     if constexpr(M::map.succ > 1)
-        pc = start_pool<K>[(M::map.n + 1) * 64 + row];
+        pc = start_pool<C>[(M::map.n + 1) * 64 + row];
     else
         pc = M::map.next;
-    return start_pool<K>[M::map.n * 64 + row];
+    return start_pool<C>[M::map.n * 64 + row];
 }
 } // namespace loom::hipvm

@@ -1251,7 +1251,8 @@ struct Taken
 /// @brief The lanes of a wave that takes threads from an input (a callable
 /// want -> Taken) until it is exhausted: their threads, and the pool of
 /// started ones behind them where the kernel and the policy use one.
-template <typename K, int P, typename RF>
+/// @p Columns: of the kernel's pool, or more (the kernel of a batch shares it).
+template <typename K, int P, typename RF, std::size_t Columns = pool_columns<K>>
 struct Lanes
 {
     static constexpr bool pooled = P == POLICY_SWEEP && StartPool<K>::used;
@@ -1323,7 +1324,7 @@ struct Lanes
                         if(w.over) break;
                     }
                     const std::uint64_t keep = ballot(spc != HALT);
-                    if(spc != HALT) pool_write<K>(s, spc, stid, rank_in(keep));
+                    if(spc != HALT) pool_write<K, Columns>(s, spc, stid, rank_in(keep));
                     // the rows are read by other lanes of this wave
                     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
                     __builtin_amdgcn_wave_barrier();
@@ -1333,7 +1334,7 @@ struct Lanes
                 const std::uint32_t g = pool < want - given ? pool : want - given;
                 if(!has && k - given < g) // k >= given for the lanes still empty
                 {
-                    tid = pool_read<K>(r, pc, row + (k - given));
+                    tid = pool_read<K, Columns>(r, pc, row + (k - given));
                     has = true;
                 }
                 row += g;

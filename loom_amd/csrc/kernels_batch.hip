@@ -19,3 +19,5 @@ LOOM_HIP_REGISTER_BATCH("pt_int_mix", S::smallpt9<float>, P::fib<std::uint64_t>,
 // integer-only batch (a smaller register file, higher occupancy)
 LOOM_HIP_REGISTER_BATCH("int_mix", P::fib<std::uint64_t>, P::collatz<std::uint64_t>,
                         P::factorial<std::uint64_t>);
+// two kernels whose START is pooled
+LOOM_HIP_REGISTER_BATCH("start_mix", P::started<std::uint64_t>, P::started<std::uint32_t>);

@@ -17,6 +17,8 @@
     X("jump4_u32", loom_amd::programs::jump4<std::uint32_t>)          \
     X("nested_u32", loom_amd::programs::nested<std::uint32_t>)        \
     X("started_u64", loom_amd::programs::started<std::uint64_t>)      \
+    X("started_u32", loom_amd::programs::started<std::uint32_t>)      \
+    X("crowded_u64", loom_amd::programs::crowded<std::uint64_t>)      \
     X("int_mix_u64", loom_amd::programs::int_mix<std::uint64_t>)      \
     X("int_mix_u32", loom_amd::programs::int_mix<std::uint32_t>)      \
     X("fp_mix_f32", loom_amd::programs::fp_mix<float>)                \

@@ -189,6 +189,64 @@ TKERNEL2(started, a, b)
     IADD(c, c, 100)
 TKERNEL_END3(s, c, d);
 
+// A long START with more words live after it than a pool may hold.
+template <std::unsigned_integral T>
+TKERNEL2(crowded, a, b)
+    IBAND(n, a, 15),
+    IMUL(r0, b, 2654435769),
+    IXOR(r0, r0, a),
+    IMUL(r1, r0, 2654435771),
+    IXOR(r1, r1, a),
+    IMUL(r2, r1, 2654435773),
+    IXOR(r2, r2, a),
+    IMUL(r3, r2, 2654435775),
+    IXOR(r3, r3, a),
+    IMUL(r4, r3, 2654435777),
+    IXOR(r4, r4, a),
+    IMUL(r5, r4, 2654435779),
+    IXOR(r5, r5, a),
+    IMUL(r6, r5, 2654435781),
+    IXOR(r6, r6, a),
+    IMUL(r7, r6, 2654435783),
+    IXOR(r7, r7, a),
+    IMUL(r8, r7, 2654435785),
+    IXOR(r8, r8, a),
+    IMUL(r9, r8, 2654435787),
+    IXOR(r9, r9, a),
+    IMUL(ra, r9, 2654435789),
+    IXOR(ra, ra, a),
+    IMUL(rb, ra, 2654435791),
+    IXOR(rb, rb, a),
+    LABEL(turn),
+    IADD(r0, r0, r5),
+    IADD(r1, r1, r6),
+    IADD(r2, r2, r7),
+    IADD(r3, r3, r8),
+    IADD(r4, r4, r9),
+    IADD(r5, r5, ra),
+    IADD(r6, r6, rb),
+    IADD(r7, r7, r0),
+    IADD(r8, r8, r1),
+    IADD(r9, r9, r2),
+    IADD(ra, ra, r3),
+    IADD(rb, rb, r4),
+    ISUB(n, n, 1),
+    IBAND(f, n, 15),
+    IPJMP2(f, done, turn),
+    LABEL(done),
+    IXOR(r0, r0, r1),
+    IXOR(r0, r0, r2),
+    IXOR(r0, r0, r3),
+    IXOR(r0, r0, r4),
+    IXOR(r0, r0, r5),
+    IXOR(r0, r0, r6),
+    IXOR(r0, r0, r7),
+    IXOR(r0, r0, r8),
+    IXOR(r0, r0, r9),
+    IXOR(r0, r0, ra),
+    IXOR(r0, r0, rb)
+TKERNEL_END2(r0, n);
+
 // Integer op mix, straight-line: every binary integer operation of the
 // contract on (a, b), folded into several outputs.
 template <std::unsigned_integral T>

@@ -53,3 +53,40 @@ def test_batch_kernels_use_no_scratch(kernels):
     spilled = {n[:60]: m["private_segment_fixed_size"] for n, m in batch
                if m["private_segment_fixed_size"]}
     assert not spilled
+
+
+def one_wave(kernels, name):
+    """The sweeping kernels of one-wave workgroups that may hold a pool of
+    started threads: (mangled name, metadata)."""
+    return [(n, m) for n, m in kernels if re.search(name, n)]
+
+
+def lds_waves(m):
+    """Waves of a SIMD that a CU's 160 KB in granules of 1280 bytes hold."""
+    return 160 * 1024 // max(1280, -(-m["group_segment_fixed_size"] // 1280) * 1280) // 4
+
+
+def test_pool_costs_no_waves(kernels):
+    """A pool of started threads takes no more LDS than its kernel's registers
+    leave waves for, however much is live after START."""
+    pooled = one_wave(kernels, r"18hybrid_pass_kernelI.*Li2ELb0ELb.E|12batch_kernelILi2E")
+    assert len(pooled) > 20
+    fewer = {}
+    for n, m in pooled:
+        by_registers = min(8, 512 // (-(-m["vgpr_count"] // 8) * 8))
+        if lds_waves(m) < by_registers:
+            fewer[n[-80:]] = (m["group_segment_fixed_size"], m["vgpr_count"])
+    assert not fewer
+
+
+def test_members_of_a_batch_share_a_pool(kernels):
+    """The batch kernel of two pooled kernels has the larger one's pool, and
+    both lookup tables."""
+    started = {n: m["group_segment_fixed_size"] for n, m in kernels
+               if "115ELc116ELc97ELc114ELc116ELc101ELc100E" in n}  # "started"
+    of = {t: max(v for n, v in started.items() if re.search(
+        rf"18hybrid_pass_kernelI.*8VariableI{t}.*Li2ELb0ELb.E", n)) for t in "jm"}
+    batch = [v for n, v in started.items() if "12batch_kernelILi2E" in n]
+    table = 32  # of a jump of four targets, aligned
+    assert len(batch) == 2 and max(batch) <= max(of.values()) + table
+    assert min(of.values()) > 1024

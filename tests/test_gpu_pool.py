@@ -23,7 +23,12 @@ def frame(n):
     return [sid, np.full(n, workloads.pt_job(61, 43, 255), np.uint32)]
 
 
-INPUTS = {"started_u64": started, "smallpt9_f32": frame}
+def crowded(n):
+    """For a kernel with too many words live after START for a pool."""
+    return started(n)
+
+
+INPUTS = {"started_u64": started, "smallpt9_f32": frame, "crowded_u64": crowded}
 FORMS = [dict(live_threshold=48), dict(live_threshold=63), dict(live_threshold=0),
          dict(live_threshold=60, waves_per_cu=1), dict(refill=False),
          dict(live_threshold=32, reconv=abi.RECONV_TOPO)]
@@ -79,3 +84,26 @@ def test_budget_holds_where_start_halts(gpu):
             assert np.array_equal(g, w), p
         for c in WORK:
             assert r.counters[c] == (base.counters[c] if p.get("stats", True) else 0), (p, c)
+
+
+@pytest.mark.parametrize("stats", [True, False])
+def test_jobs_share_a_pool(gpu, stats):
+    """Jobs of two pooled kernels in one batch, one and many pools long: a
+    wave that goes from one kernel's job to the other's uses the same LDS."""
+    kernels = ("started_u64", "started_u32")
+    for rows in ((1, 63, 64, 65, 129, 1000), (40000, 7, 30011, 500)):
+        b, keep = loom_amd.Batch("start_mix"), []
+        for i, n in enumerate(rows):
+            for name in kernels:
+                ins = [c.astype(dt) for c, dt in zip(started(n + i), loom_amd.kernel(name).inputs)]
+                want, _ = O.run(name, ins)
+                outs = [loom_amd.DeviceArray(n + i, dt) for dt in loom_amd.kernel(name).outputs]
+                b.add(name, [loom_amd.DeviceArray.from_numpy(c) for c in ins], outs)
+                keep.append((name, n + i, outs, want))
+        for waves in (1, 0):
+            print(f"[gpu] batch of pooled kernels {rows} stats {stats} waves {waves}", flush=True)
+            b.run(loom_amd.make_params(mode=abi.MODE_HYBRID, stats=stats, waves_per_cu=waves))
+            for name, n, outs, want in keep:
+                for g, w in zip(outs, want):
+                    assert np.array_equal(g.numpy(), w), (name, n, waves)
+                    g.zero()
