@@ -135,13 +135,14 @@ fma_(T x, T y, T z)
 }
 
 /// @brief Correctly rounded f32 square root of x = ±0 or 2^-96 <= x < inf from
-/// the hardware's reciprocal root y (within one ulp): s = x·y, corrected by
-/// its residual, s + (x - s²)·y/2.  The residual is exact in one fma down to
-/// x = 2^-100, so what is rounded last is off by about 2^-46, and no root of a
-/// 24-bit number lies that near a rounding boundary unless it is hit by all
-/// values of two binades, which were compared one by one with the compiler's
-/// root (all of [2^-96, max] was: no difference).  For x = ±0, whose root is
-/// x·y, y is kept finite by a maximum of the bits as signed integers.
+/// the hardware's reciprocal root y: s = x·y, corrected by its residual,
+/// s + (x - s²)·y/2.  That the last rounding gives the nearest root is a
+/// property of this hardware's estimates and of every single x, not of their
+/// stated accuracy: for x = 0x406E9372 an estimate 0.85 ulp high, within the
+/// stated one, would give the neighbour of the root.  All of [2^-96, inf) is
+/// compared with the correctly rounded root in tests/test_roots.py.  For
+/// x = ±0, whose root is x·y, y is kept finite by a maximum of the bits as
+/// signed integers.
 template <bool Zero>
 LOOM_DEVICE float
 sqrt_refined(float x)
@@ -158,9 +159,10 @@ sqrt_refined(float x)
 }
 
 /// @brief Correctly rounded 1/d of a normal |d| <= 2^124: the hardware's
-/// estimate (within one ulp) and one Newton step, which rounds correctly for
-/// each of the 2^23 mantissas (compared one by one with the compiler's
-/// quotient; the estimate's mantissa does not depend on the exponent).
+/// estimate, whose mantissa does not depend on the exponent, and one Newton
+/// step.  As for the root, that this rounds correctly is a property of the
+/// estimates: each of the 2^23 mantissas is compared in tests/test_roots.py
+/// (as a root's reciprocal).
 LOOM_DEVICE float
 rcp_refined(float d)
 {

@@ -29,7 +29,7 @@ def special(dt):
                     dtype=dt)
 
 
-def inputs(kind, groups=48, seed=31):
+def inputs(kind, groups=72, seed=31):  # every special value once
     dt, ut = KINDS[kind]
     rng = np.random.default_rng(seed)
     bits = 32 if dt is np.float32 else 64
@@ -38,7 +38,7 @@ def inputs(kind, groups=48, seed=31):
     for g in range(groups):
         if g % 3 == 0:
             # positive, normal, exponent spread over the fast range
-            e = rng.uniform(-90, 120, WAVE)
+            e = rng.uniform(-95, 127, WAVE)
             v = (rng.uniform(1, 2, WAVE) * 2.0 ** e).astype(dt)
         elif g % 3 == 1:
             e = rng.uniform(-90, 120, WAVE)
@@ -77,8 +77,11 @@ def test_inputs_reach_both_branches(kind):
     g = x.reshape(-1, WAVE)
     dt = x.dtype.type
     with np.errstate(invalid="ignore"):
-        fast = ((g >= dt(2.0 ** -96)) & (g <= dt(2.0 ** 126))).all(axis=1)
-    assert fast.sum() >= 10 and (~fast).sum() >= 10
+        fast = (g >= dt(2.0 ** -96)) & (g < dt(np.inf))
+    # the square root's branch takes zeros too, the reciprocal's does not
+    for ok in (fast, fast | (g == 0)):
+        assert ok.all(axis=1).sum() >= 10 and (~ok.all(axis=1)).sum() >= 10
+    assert ((fast | (g == 0)).all(axis=1) & ~fast.all(axis=1)).sum() >= 2
 
 
 @pytest.mark.parametrize("kind", ["f32", "f64"])
@@ -119,3 +122,43 @@ def test_gpu_roots(gpu, kind, mode):
         got = d.numpy()
         ok = same(got, want)
         assert ok.all(), (fn, kind, mode, x[~ok][:4], got[~ok][:4], want[~ok][:4])
+
+
+@pytest.mark.gpu
+def test_gpu_every_root_of_the_fast_range(gpu):
+    """The device's fast f32 roots are correctly rounded because of what its
+    estimates are, not of what is promised of them, so each is looked at: every
+    float of [2^-96, inf), two binades at a time.  Their roots are those of
+    [1, 4) scaled by a power of two, exactly, and reach every mantissa, so the
+    reciprocals are those of every mantissa too."""
+    import loom_amd
+    from loom_amd import abi
+    base = np.arange(0x3F800000, 0x40800000, dtype=np.uint32)  # [1, 4)
+    s, r = (w.view(np.uint32) for w in expected(base.view(np.float32)))
+    assert len(np.unique(s & 0x7FFFFF)) == 1 << 23
+    k = loom_amd.kernel("roots_f32")
+    out = [loom_amd.DeviceArray(len(base), np.float32) for _ in range(2)]
+    for e in range(-48, 64):  # 4^e
+        x = base + np.uint32(2 * e << 23 & 0xFFFFFFFF)
+        din = [loom_amd.DeviceArray.from_numpy(x.view(np.float32))]
+        # large runs without statistics take four threads a lane, others one
+        loom_amd.run(k, abi.MODE_COMPACT, din, out, params=loom_amd.make_params(stats=e % 2 == 0))
+        if e % 16 == 0:
+            print(f"[gpu] roots of [2^{2 * e}, 2^{2 * e + 2})", flush=True)
+        for d, want, step in zip(out, (s, r), (e, -e)):
+            bad = d.numpy().view(np.uint32) != want + np.uint32(step << 23 & 0xFFFFFFFF)
+            assert not bad.any(), (e, step, x[bad][:4])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("e", [-48, 0, 63])
+def test_gpu_roots_of_zeros_among_others(gpu, e):
+    """A zero in an otherwise fast wave: the square root's branch stays."""
+    import loom_amd
+    from loom_amd import abi
+    x = (np.random.default_rng(e + 50).integers(0x3F800000, 0x40800000, 1 << 16, dtype=np.uint32) +
+         np.uint32(2 * e << 23 & 0xFFFFFFFF)).view(np.float32)
+    x[7::64], x[40::128] = 0.0, -0.0
+    r = loom_amd.run("roots_f32", abi.MODE_COMPACT, [x])
+    for got, want in zip(r.outputs, expected(x)):
+        assert (got.view(np.uint32) == want.view(np.uint32)).all()
