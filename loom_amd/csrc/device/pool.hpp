@@ -24,7 +24,14 @@
 namespace loom::hipvm
 {
 /// Operations of a START worth pooling.  Below, reading the pool costs about
-/// what START does (fib and Collatz: 3 operations, the cubic: 4).
+/// what START does (fib and Collatz with 3 operations, pooled: 2-14% slower;
+/// the cubic with 4: even).  From 26 to 98 operations the pool pays where the
+/// threads do work between refills: loops of 32 or 68 operations and 1 to 32
+/// trips, refilled at 48 lanes, took 0.68 to 0.96 of the time without it
+/// (12,000,003 threads; 3,000,017: 0.86 to 1.00; 200,003, where few refills
+/// happen: 0.98 to 1.04).  Where the columns are the cost (8 operations and a
+/// few trips) it is up to 10% slower, at 26 as at 98 operations; trip counts
+/// are not known here.
 inline constexpr std::uint32_t kPoolMinOps = 24;
 
 /// @brief 32-bit words of the registers in @p live.
