@@ -3,6 +3,8 @@ from run to run, counters that are subtracted instead of cleared, error words
 in host memory, pinned columns of small host calls.  Runs of different forms,
 with and without statistics, failing ones among them, in one sequence: every
 result and every count is that of the run alone."""
+import ctypes as C
+
 import numpy as np
 import pytest
 
@@ -45,9 +47,11 @@ def test_sequence_of_runs(gpu):
                     ctx.run("fib_u64", abi.MODE_HYBRID, [din], [out], params=p)
                 continue
             if form == "batch":
-                b = loom_amd.Batch("int_mix")
+                b, r = loom_amd.Batch("int_mix"), abi.RunStats()
                 b.add("fib_u64", [din], [out])
-                r = b.run(loom_amd.make_params(mode=abi.MODE_HYBRID, stats=stats))
+                p = loom_amd.make_params(mode=abi.MODE_HYBRID, stats=stats)
+                abi.check(abi.load().loom_ctx_batch_run(ctx.handle, b.set, b._table(), 1,
+                                                        C.byref(p), C.byref(r)), "batch")
             else:
                 m = abi.MODE_HYBRID if form == "hybrid" else abi.MODE_COMPACT
                 r = ctx.run("fib_u64", m, [din], [out],
