@@ -170,7 +170,10 @@ int loom_kernel_dump(int kernel, char* buf, size_t len, size_t* needed);
  * LOOM_RESOURCES_REGROUP for the hybrid pass kernel that regroups, which a
  * run with loom_params.regroup set launches; runs without it launch a pass
  * kernel compiled without the queue paths; or'ed with LOOM_RESOURCES_MEMORY
- * for the compact kernel whose register file is in device memory). */
+ * for the compact kernel whose register file is in device memory).  They are
+ * those of the builds that runs with statistics launch; the builds for runs
+ * that count no work (sweeps of regions, several threads a lane) are not
+ * reported. */
 #define LOOM_RESOURCES_REGROUP 0x100
 #define LOOM_RESOURCES_MEMORY 0x200
 #define LOOM_RESOURCES_WORKGROUP 0x400 /* the workgroup-regrouping kernel (reconv 0 or 2) */

@@ -176,7 +176,10 @@ def make_params(threshold=0, live_threshold=None, refill=True, regroup=False, wa
     registers in device memory (sweep policy); `regroup` = REGROUP_WORKGROUP
     sorts a workgroup's threads by block between run phases of
     `regroup_phase` dispatches, in workgroups of `regroup_waves` waves (16,
-    one per CU, or 8, two per CU; 0 = 16)."""
+    one per CU, or 8, two per CU; 0 = 16).  `stats` collects the run's
+    counters, which active_lane_fraction needs; without them and with the
+    default `max_steps`, kernels with blocks below eight operations sweep
+    regions of blocks (Collatz: half the time)."""
     p = abi.Params()
     if reconv is None:
         reconv = abi.RECONV_SUCCESSOR_MAJOR if mode == abi.MODE_COMPACT else abi.RECONV_SWEEP
@@ -277,7 +280,9 @@ class Context:
 
 class compact_function:
     """Predicated wave64 form (reference simd::compact_function<K>,
-    src/vm/simd.hpp:4329-4335): `f(*inputs)` returns the output columns."""
+    src/vm/simd.hpp:4329-4335): `f(*inputs)` returns the output columns.
+    `f.last` is the run's result; its counters cost time, and `stats=False`
+    leaves them out (make_params)."""
 
     mode = abi.MODE_COMPACT
 
@@ -297,7 +302,8 @@ class hybrid_function(compact_function):
     (the reference UTRt·N, simd.hpp:4094-4098), `refill` admits new threads
     into free lanes when at most `live_threshold` lanes are live, `regroup`
     spills survivors to per-label queues once no input is left,
-    `waves_per_cu` sizes the persistent grid."""
+    `waves_per_cu` sizes the persistent grid; `stats=False` runs the build
+    that counts no work (Collatz: half the time)."""
 
     mode = abi.MODE_HYBRID
 

@@ -184,7 +184,7 @@ outside_root_range(float x)
 /// active lane's x allows it: a wave-uniform branch, no per-lane divergence.
 /// The compiler's sequence is 16 instructions; refining v_sqrt by its two
 /// neighbours, which this replaced, was 9 and 2 (path-traced 1024x768x64 frame
-/// 7.50 ms with it, 7.26 with this).
+/// 7.50 ms with it, 7.24 with this).
 LOOM_DEVICE float
 sqrt_rn(float x)
 {

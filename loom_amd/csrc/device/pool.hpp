@@ -11,7 +11,7 @@
 /// from there.  Registers that START sets to a literal are set again at the
 /// refill instead.  Threads that halt in START never enter the pool.
 ///
-/// The path tracer's 1024x768x64 frame: 7.24 ms without the pool (refilled at 48
+/// The path tracer's 1024x768x64 frame: 7.18 ms without the pool (refilled at 48
 /// lanes, 72% of the lanes active), 6.44 with it (refilled at 60, 81%).
 ///
 /// Used where it pays: START of at least kPoolMinOps operations that no other

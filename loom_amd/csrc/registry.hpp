@@ -95,6 +95,7 @@ launch_batch(const CtlArgs& c, const BatchArgs& a, unsigned grid, hipStream_t s)
                           launch(batch_kernel<P, true, Ks...>, grid, 64, s, c, a);
 }
 
+/// As hybrid_occupancy: of the counted build.
 template <int P, typename... Ks>
 int
 batch_occupancy()
@@ -238,6 +239,9 @@ launch_hybrid_pass(const IoArgs& io, const CtlArgs& c, const HybridArgs& h, unsi
     return launch(hybrid_pass_kernel<K, P, false>, grid, 64, s, io, c, h);
 }
 
+/// Resident one-wave workgroups per CU of the counted build.  The one that
+/// counts no work needs no more registers in any kernel here, so a grid of this
+/// size is resident with either.
 template <typename K, int P>
 int
 hybrid_occupancy(bool regroup)
@@ -253,7 +257,7 @@ hybrid_occupancy(bool regroup)
 }
 
 /// @brief Registers and scratch of the compiled kernel of @p mode and
-/// @p policy (LOOM_MODE_COMPACT: the predicated kernel, with its register
+/// @p policy, in its counted build (LOOM_MODE_COMPACT: the predicated kernel, with its register
 /// file in memory under LOOM_RESOURCES_MEMORY; LOOM_MODE_HYBRID: the pass
 /// kernel, with the regroup paths under LOOM_RESOURCES_REGROUP).
 template <typename K>
